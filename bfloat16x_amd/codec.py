@@ -49,24 +49,21 @@ def _quantize_device(w: torch.Tensor) -> dict:
     delta = torch.empty(stream_words(n, 3), **i32)
     emax = torch.empty((n + SUB - 1) // SUB, dtype=torch.uint8, device=dev)
     ws = torch.empty((int(L.bf16x_encode_workspace(out_f, in_f)) + 15) // 16 * 4, **i32)
-    n_ovf = torch.zeros(1, dtype=torch.int64, device=dev)
-    cap = max(1, n // 8)
+    n_ovf = torch.empty(1, dtype=torch.int64, device=dev)
     stream = _lib.stream_of(dev)
-    for _ in range(2):
-        idx = torch.empty(cap, **i32)
-        val = torch.empty(cap, dtype=torch.uint8, device=dev)
-        st = L.bf16x_encode(bits.data_ptr(), out_f, in_f, SUB, sign.data_ptr(), sign.numel(), mant.data_ptr(),
-                            mant.numel(), delta.data_ptr(), delta.numel(), emax.data_ptr(), emax.numel(),
-                            idx.data_ptr(), val.data_ptr(), cap, n_ovf.data_ptr(), ws.data_ptr(),
-                            ws.numel() * 4, stream)
-        _lib.check(st, "bf16x_encode")
-        k = int(n_ovf.item())
-        if k <= cap:
-            break
-        cap = k
-    return dict(emax=emax, sign_packed=sign, mant_packed=mant, delta_packed=delta,
-                delta_ovf_idx=idx[:k].clone(), delta_ovf_val=val[:k].clone(),
-                out_f=out_f, in_f=in_f, sub=SUB)
+    st = L.bf16x_encode_streams(bits.data_ptr(), out_f, in_f, SUB, sign.data_ptr(), sign.numel(), mant.data_ptr(),
+                                mant.numel(), delta.data_ptr(), delta.numel(), emax.data_ptr(), emax.numel(),
+                                n_ovf.data_ptr(), ws.data_ptr(), ws.numel() * 4, stream)
+    _lib.check(st, "bf16x_encode_streams")
+    k = int(n_ovf.item())
+    idx = torch.empty(k, **i32)
+    val = torch.empty(k, dtype=torch.uint8, device=dev)
+    if k:
+        st = L.bf16x_encode_table(bits.data_ptr(), out_f, in_f, idx.data_ptr(), val.data_ptr(), k, ws.data_ptr(),
+                                  ws.numel() * 4, stream)
+        _lib.check(st, "bf16x_encode_table")
+    return dict(emax=emax, sign_packed=sign, mant_packed=mant, delta_packed=delta, delta_ovf_idx=idx,
+                delta_ovf_val=val, out_f=out_f, in_f=in_f, sub=SUB)
 
 
 def bf16x_quantize(w: torch.Tensor, sub: int = SUB, n_threads: int = 0) -> dict:

@@ -99,8 +99,17 @@ int bf16x_encode_host(const uint16_t* w_bits, int64_t out_f, int64_t in_f, int32
  * outputs and a workspace of bf16x_encode_workspace bytes (16-byte aligned).
  * The table count is written to *n_ovf (device int64); entries past ovf_cap
  * are not written, so a caller whose cap was short re-runs with a larger one.
- * Streams have at least bf16x_stream_words(N, b) words. */
+ * Streams have at least bf16x_stream_words(N, b) words.
+ * bf16x_encode_streams writes all but the table; bf16x_encode_table then
+ * writes the table from the same weight and workspace (same stream, workspace
+ * untouched in between), so a caller can size it by *n_ovf. */
 int64_t bf16x_encode_workspace(int64_t out_f, int64_t in_f);
+int bf16x_encode_streams(const uint16_t* w_bits, int64_t out_f, int64_t in_f, int32_t sub,
+                         int32_t* sign, int64_t n_sign, int32_t* mant, int64_t n_mant, int32_t* delta,
+                         int64_t n_delta, uint8_t* emax, int64_t n_emax, int64_t* n_ovf, void* workspace,
+                         int64_t workspace_bytes, bf16x_stream_t stream);
+int bf16x_encode_table(const uint16_t* w_bits, int64_t out_f, int64_t in_f, int32_t* ovf_idx, uint8_t* ovf_val,
+                       int64_t ovf_cap, const void* workspace, int64_t workspace_bytes, bf16x_stream_t stream);
 int bf16x_encode(const uint16_t* w_bits, int64_t out_f, int64_t in_f, int32_t sub,
                  int32_t* sign, int64_t n_sign, int32_t* mant, int64_t n_mant, int32_t* delta, int64_t n_delta,
                  uint8_t* emax, int64_t n_emax, int32_t* ovf_idx, uint8_t* ovf_val, int64_t ovf_cap,

@@ -81,3 +81,25 @@ def test_device_encoder_config_shapes(bx, shape):
     plan = bx.build_plan_host(dd, device=DEV)
     dec = bx.bf16x_decode(dd["sign_packed"], dd["mant_packed"], dd["delta_packed"], dd["emax"], *shape, plan=plan)
     assert torch.equal(dec.view(torch.int16).cpu(), w.view(torch.int16))
+
+
+def spread_bits(shape, seed):
+    """Exponents uniform over 100 .. 135: most elements are in the table, so
+    the table kernel takes every segment from the weight."""
+    rng = np.random.default_rng(seed)
+    return ((rng.integers(0, 2, size=shape) << 15) | (rng.integers(100, 136, size=shape) << 7)
+            | rng.integers(0, 128, size=shape)).astype(np.uint16)
+
+
+# a wave's 64 atoms (2048 elements) and a workgroup's 256, one element either
+# side; more than one iteration per wave (N > 2^25), the last one ragged
+@pytest.mark.parametrize("shape", [(1, 2047), (1, 2048), (1, 2049), (1, 8191), (1, 8193), (3, 2731), (65, 32),
+                                   (8200, 4101)])
+@pytest.mark.parametrize("kind", ["bench", "spread", "flat"])
+def test_device_encoder_segments(bx, shape, kind):
+    bits = {"bench": lambda: dc.bench_weight_bits(*shape, seed=5), "spread": lambda: spread_bits(shape, 6),
+            "flat": lambda: np.full(shape, 0x3C00, np.uint16)}[kind]()       # flat: an empty table
+    w = torch.from_numpy(bits.view(np.int16).copy()).view(torch.bfloat16)
+    d = bx.bf16x_quantize(w.to(DEV))
+    same_dict(d, bx.bf16x_quantize(w), (kind, shape))
+    assert (d["delta_ovf_idx"].numel() == 0) == (kind == "flat")
