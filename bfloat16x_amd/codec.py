@@ -184,11 +184,67 @@ def _host_i32(t) -> torch.Tensor:
     return t.detach().cpu().contiguous()
 
 
+def _on_device(packed: dict, device) -> bool:
+    """Whether the dict is one the device builder takes as it stands: every
+    tensor in the dict's own types and full lengths on `device`, a table,
+    positions in int32."""
+    if device is None:
+        return False
+    dev = torch.device(device)
+    if dev.type != "cuda":
+        return False
+    if dev.index is None:
+        dev = torch.device("cuda", torch.cuda.current_device())
+    types = dict.fromkeys(("sign_packed", "mant_packed", "delta_packed", "delta_ovf_idx"), torch.int32)
+    types.update(emax=torch.uint8, delta_ovf_val=torch.uint8)
+    for k, dt in types.items():
+        t = packed[k]
+        if not isinstance(t, torch.Tensor) or t.device != dev or t.dtype != dt:
+            return False
+    out_f, in_f = int(packed["out_f"]), int(packed["in_f"])
+    n, N = packed["delta_ovf_idx"].numel(), out_f * in_f
+    return (0 < n == packed["delta_ovf_val"].numel() and out_f > 0 and 0 < N <= 2 ** 31 - 1
+            and packed["emax"].numel() >= -(-N // SUB)
+            and all(packed[k].numel() >= stream_words(N, b)
+                    for k, b in (("sign_packed", 1), ("mant_packed", 7), ("delta_packed", 3))))
+
+
+def _build_plan_on_device(packed: dict) -> Bf16xPlan:
+    """build_plan_host (check = 1) of a dict on the GPU, built there."""
+    out_f, in_f = int(packed["out_f"]), int(packed["in_f"])
+    sign, mant, delta, emax, idx, val = (packed[k].detach().contiguous() for k in (
+        "sign_packed", "mant_packed", "delta_packed", "emax", "delta_ovf_idx", "delta_ovf_val"))
+    dev, n = sign.device, idx.numel()
+    L = _lib.lib()
+    stream = _lib.stream_of(dev)
+    ws = torch.empty(int(L.bf16x_plan_device_workspace(n)) // 4, dtype=torch.int32, device=dev)
+    count = torch.empty(1, dtype=torch.int64, device=dev)
+    st = L.bf16x_plan_device_count(idx.data_ptr(), val.data_ptr(), n, delta.data_ptr(), delta.numel(),
+                                   emax.data_ptr(), emax.numel(), out_f, in_f, count.data_ptr(), ws.data_ptr(),
+                                   ws.numel() * 4, stream)
+    _lib.check(st, "bf16x_plan_host")
+    tile_off = torch.empty(plan_tiles(out_f, in_f) + 1, dtype=torch.int32, device=dev)
+    k = int(count.item())
+    if k < 0:
+        raise _lib.Bf16xError(_lib.ETABLE, "bf16x_plan_host")
+    tile_ent = torch.empty(max(k, 1), dtype=torch.int32, device=dev)
+    tile_sat = torch.empty(max(k, 1), dtype=torch.uint8, device=dev)
+    st = L.bf16x_plan_device_write(idx.data_ptr(), val.data_ptr(), n, sign.data_ptr(), sign.numel(), mant.data_ptr(),
+                                   mant.numel(), emax.data_ptr(), emax.numel(), out_f, in_f, k, tile_off.data_ptr(),
+                                   tile_ent.data_ptr(), tile_sat.data_ptr(), ws.data_ptr(), ws.numel() * 4, stream)
+    _lib.check(st, "bf16x_plan_host")
+    return Bf16xPlan(tile_off, tile_ent, tile_sat, k, out_f, in_f)
+
+
 def build_plan_host(packed: dict, check: int = 1, device=None) -> Bf16xPlan:
-    """Plan from a (host) packed dict with the C++ builder; moved to `device`."""
+    """Plan from a packed dict, on `device` (the host when None).  A dict whose
+    tensors are on `device` already is planned there (bf16x_plan_device_*, the
+    same checks and the same plan); others by the C++ builder on the host."""
     out_f, in_f = int(packed["out_f"]), int(packed["in_f"])
     if int(packed.get("sub", SUB)) != SUB:
         raise _lib.Bf16xError(_lib.ESUB, "build_plan_host")
+    if check == 1 and _on_device(packed, device):
+        return _build_plan_on_device(packed)
     sign = _host_i32(packed["sign_packed"])
     mant = _host_i32(packed["mant_packed"])
     delta = _host_i32(packed["delta_packed"])

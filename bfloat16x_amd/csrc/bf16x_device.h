@@ -277,4 +277,16 @@ __device__ __forceinline__ float wave_sum(float v) {
   return v;
 }
 
+// exclusive prefix over the wave's lanes, and the wave's total
+__device__ __forceinline__ uint32_t wave_prefix(uint32_t c, int lane, uint32_t& total) {
+  uint32_t s = c;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t u = __shfl_up(s, o, 64);
+    if (lane >= o) s += u;
+  }
+  total = __builtin_amdgcn_readlane(s, 63);
+  return s - c;
+}
+
 }  // namespace bf16x

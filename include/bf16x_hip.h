@@ -132,6 +132,23 @@ int bf16x_plan_host(const int32_t* ovf_idx, const uint8_t* ovf_val, int64_t n_ov
                     uint32_t* tile_off, uint32_t* tile_ent, uint8_t* tile_sat, int64_t ent_cap,
                     int64_t* n_fix);
 
+/* Device plan builder: bf16x_plan_host (check = 1) for a dict in device
+ * memory, n_ovf > 0 entries, out_f * in_f below 2^31.  _count checks the table
+ * and writes the number of entries the plan keeps to *n_fix (device int64), or
+ * -1 where bf16x_plan_host returns BF16X_ETABLE; _write, given that number
+ * (>= 0) and the same table and workspace (same stream, workspace untouched in
+ * between), writes tile_off [out_f * tiles_per_row + 1] and n_fix entries.
+ * Workspace: bf16x_plan_device_workspace(n_ovf) bytes, 4-byte aligned. */
+int64_t bf16x_plan_device_workspace(int64_t n_ovf);
+int bf16x_plan_device_count(const int32_t* ovf_idx, const uint8_t* ovf_val, int64_t n_ovf, const int32_t* delta,
+                            int64_t n_delta, const uint8_t* emax, int64_t n_emax, int64_t out_f, int64_t in_f,
+                            int64_t* n_fix, void* workspace, int64_t workspace_bytes, bf16x_stream_t stream);
+int bf16x_plan_device_write(const int32_t* ovf_idx, const uint8_t* ovf_val, int64_t n_ovf, const int32_t* sign,
+                            int64_t n_sign, const int32_t* mant, int64_t n_mant, const uint8_t* emax,
+                            int64_t n_emax, int64_t out_f, int64_t in_f, int64_t n_fix, uint32_t* tile_off,
+                            uint32_t* tile_ent, uint8_t* tile_sat, const void* workspace, int64_t workspace_bytes,
+                            bf16x_stream_t stream);
+
 /* ------------------------------------------------------------------------
  * Device plan from the reference's per-row CSR (olk col int32, old true
  * delta int32, oloff int32 [out_f + 1]) -- the arguments of
