@@ -112,13 +112,14 @@ def gemm_kernel_name(M: int, out_f: int, in_f: int) -> str:
         return "gemm_rows_kernel (rows streamed as in the GEMV, 16x16x32 MFMA)"
     if ops._use_chunks(M, out_f, in_f, torch.device("cuda:0")):
         return "gemm_chunks_kernel (rows streamed in column chunks, 16x16x32 MFMA)"
-    if M <= 64 and in_f % 128 == 0:
+    ws4 = in_f % 256 == 0 and (M > 64 or (M > 32 and out_f * in_f >= 1 << 25))
+    if M <= 64 and in_f % 128 == 0 and not ws4:
         return "gemm_skinny2_kernel (16x16x32 MFMA, few rows)"
     if M <= 32:
         return "gemm_skinny_kernel"
+    if ws4:
+        return "gemm_ws4_kernel (wave-specialised, 256-column groups, 32x32x16 MFMA)"
     if M >= 192:
-        if (in_f // 64) % 4 == 0:
-            return "gemm_ws4_kernel (wave-specialised, 256-column groups, 32x32x16 MFMA)"
         return "gemm_ws_kernel (wave-specialised, 32x32x16 MFMA)"
     return "gemm_kernel (tiled)"
 

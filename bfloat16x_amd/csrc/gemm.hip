@@ -510,14 +510,30 @@ int64_t skinny2_rows() {
   return r < 0 ? 0 : (r > 64 ? 64 : r);
 }
 
-bool use_skinny2(int64_t M, int64_t in_f) { return M <= skinny2_rows() && in_f % 128 == 0; }
 
-// Smallest M served by the wave-specialised kernel (256-row tiles).
-int64_t ws_rows() {
+// Smallest M served by the wave-specialised kernel.  In four-step groups
+// (in_f % 256 == 0) it has 64- and 128-token tiles: past the few-row kernels'
+// 64 rows it is faster than the tiled kernel at every shape measured (65 rows,
+// us: 14336x4096 42.8 against 63.2, 4096x4096 22.7 against 28.8, 3072x1024
+// 15.0 against 16.2, 1024x4096 18.6 against 18.5), and from 33 rows faster than
+// the 16x16x32 kernel once the weight is large (33 / 64 rows: 4096x14336 39.0
+// / 39.3 against 43.1 / 45.7, 8192x8192 40.5 / 40.8 against 42.7 / 50.6;
+// 6144x4096 24.8 / 25.1 against 22.2 / 25.1).  One step at a time it has the
+// 256-token tile only.
+constexpr int64_t kWsFewRowsMin = 33, kWsFewRowsElems = (int64_t)1 << 25;
+bool ws_groups(int64_t in_f) { return in_f % 256 == 0 && tuning(BF16X_TUNE_GEMM_WS_GROUPED) != 0; }
+int64_t ws_rows(int64_t in_f) {
   const int64_t t = tuning(BF16X_TUNE_GEMM_WS_MIN_ROWS);
-  return t >= 0 ? t : 192;
+  return t >= 0 ? t : (ws_groups(in_f) ? 65 : 192);
+}
+bool ws_few_rows(int64_t M, int64_t out_f, int64_t in_f) {
+  return M >= kWsFewRowsMin && out_f * in_f >= kWsFewRowsElems && ws_groups(in_f) &&
+         tuning(BF16X_TUNE_GEMM_WS_MIN_ROWS) < 0 && tuning(BF16X_TUNE_GEMM_SKINNY2_MAX) < 0;
 }
 
+bool use_skinny2(int64_t M, int64_t out_f, int64_t in_f) {
+  return M <= skinny2_rows() && in_f % 128 == 0 && !ws_few_rows(M, out_f, in_f);
+}
 
 // Largest M served by the few-row kernel (at most 128, its column-block
 // limit; measured faster than the tiled kernel up to 32 rows).
@@ -528,7 +544,10 @@ int64_t skinny_rows() {
 }
 
 // M >= ws_rows() and past both few-row kernels
-bool use_ws(int64_t M, int64_t in_f) { return M >= ws_rows() && !use_skinny2(M, in_f) && M > skinny_rows(); }
+bool use_ws(int64_t M, int64_t out_f, int64_t in_f) {
+  return ws_few_rows(M, out_f, in_f) ||
+         (M >= ws_rows(in_f) && !use_skinny2(M, out_f, in_f) && M > skinny_rows());
+}
 
 struct GemmShape {
   int bm;        // rows of x per tile
@@ -566,9 +585,9 @@ GemmShape gemm_shape(int64_t M, int64_t out_f, int64_t in_f) {
 
 extern "C" int64_t bf16x_gemm_workspace(int64_t M, int64_t out_f, int64_t in_f) {
   if (M <= 0 || out_f <= 0 || in_f < kBK) return 0;
-  if (use_skinny2(M, in_f)) return bf16x_gemm_skinny2_workspace(M, out_f, in_f);
+  if (use_skinny2(M, out_f, in_f)) return bf16x_gemm_skinny2_workspace(M, out_f, in_f);
   if (M <= skinny_rows()) return 0;
-  if (use_ws(M, in_f)) return bf16x_gemm_ws_workspace(M, out_f, in_f);
+  if (use_ws(M, out_f, in_f)) return bf16x_gemm_ws_workspace(M, out_f, in_f);
   const GemmShape g = gemm_shape(M, out_f, in_f);
   return g.nsplit > 1 ? (int64_t)g.nsplit * M * out_f * 4 : 0;
 }
@@ -591,7 +610,7 @@ extern "C" int bf16x_gemm(const void* x, int32_t x_dtype, int64_t M, const int32
   if (!aligned4(sign) || !aligned4(mant) || !aligned4(delta) || !aligned2(emax) || !aligned16(x) || !aligned4(y))
     return BF16X_EARG;
   hipStream_t st = (hipStream_t)stream;
-  if (use_skinny2(M, in_f)) {
+  if (use_skinny2(M, out_f, in_f)) {
     rc = bf16x_gemm_skinny2_launch((const uint16_t*)x, M, (const uint32_t*)sign, (const uint32_t*)mant,
                                    (const uint32_t*)delta, (const uint16_t*)emax, kp_off, kp_ent, out_f, in_f,
                                    mode == BF16X_EXACT, y_dtype == BF16X_F32, y, workspace, workspace_bytes, st);
@@ -603,7 +622,7 @@ extern "C" int bf16x_gemm(const void* x, int32_t x_dtype, int64_t M, const int32
                                   mode == BF16X_EXACT, y_dtype == BF16X_F32, y, st);
     return rc ? rc : launch_status();
   }
-  if (use_ws(M, in_f)) {
+  if (use_ws(M, out_f, in_f)) {
     rc = bf16x_gemm_ws_launch((const uint16_t*)x, M, (const uint32_t*)sign, (const uint32_t*)mant,
                               (const uint32_t*)delta, (const uint16_t*)emax, nullptr, kp_off, kp_ent, out_f, in_f,
                               mode == BF16X_EXACT, y_dtype == BF16X_F32, y, workspace, workspace_bytes, st);

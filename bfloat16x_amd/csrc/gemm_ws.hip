@@ -17,7 +17,8 @@
 //    130-220 B/clk for 16-byte reads.  Register budget (two waves per SIMD,
 //    256 registers each) limits an MFMA wave to 128 accumulators.
 //
-// A workgroup is 8 waves and owns an output tile of 256 x rows (tokens) by 128
+// A workgroup is 8 waves (12 for the smaller tiles of the grouped kernel) and
+// owns an output tile of 256 x rows (tokens) by 128
 // W rows over a range of 64-column K steps (all of K, or one split of it when
 // the tile count alone leaves CUs idle; split partials are fp32 and summed in
 // split order by a second kernel).
@@ -142,34 +143,36 @@ __device__ __forceinline__ WsWork ws_work(const WsGrid& g, int units) {
 // The output tile from the MFMA waves' accumulators: register v of lane l ->
 // token row 8(v/4) + 4(l/32) + v%4, W row l%32.  A split tile's partial goes
 // to its own BM x 128 fp32 tile of `part` (all of it: rows past M and
-// columns past out_f hold zeros), in K-range order.  NI: 32-token tiles per
-// wave (the wave owns tokens NI 32 wave .. + NI 32 - 1 of the tile).
-template <bool YF32, int NI = 2>
-__device__ __forceinline__ void ws_store(const f32x16 (&acc)[NI][4], const WsWork& w, int wave, int lane, int64_t M,
+// columns past out_f hold zeros), in K-range order.  The wave owns NT 32-token
+// tiles from token 32 NT (wave % TG) and NJ 32-row W tiles from row
+// 32 NJ (wave / TG).
+template <bool YF32, int NT, int TG, int NJ>
+__device__ __forceinline__ void ws_store(const f32x16 (&acc)[NT][NJ], const WsWork& w, int wave, int lane, int64_t M,
                                          int64_t out_f, int ltiles, void* __restrict__ y, float* __restrict__ part) {
-  constexpr int BM = 4 * 32 * NI;
+  constexpr int BM = 32 * NT * TG;
   const int lr = lane & 31, h = lane >> 5;
+  const int t0 = 32 * NT * (wave % TG), r0 = 32 * NJ * (wave / TG);
   if (w.lt >= 0) {
     float* pt = part + ((int64_t)w.kb * ltiles + w.lt) * (BM * kBN);
 #pragma unroll
-    for (int i = 0; i < NI; ++i)
+    for (int i = 0; i < NT; ++i)
 #pragma unroll
-      for (int jj = 0; jj < 4; ++jj)
+      for (int jj = 0; jj < NJ; ++jj)
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
-          const int r = wave * 32 * NI + i * 32 + 8 * (v >> 2) + 4 * h + (v & 3);
-          pt[r * kBN + jj * 32 + lr] = acc[i][jj][v];
+          const int r = t0 + i * 32 + 8 * (v >> 2) + 4 * h + (v & 3);
+          pt[r * kBN + r0 + jj * 32 + lr] = acc[i][jj][v];
         }
     return;
   }
 #pragma unroll
-  for (int i = 0; i < NI; ++i) {
+  for (int i = 0; i < NT; ++i) {
 #pragma unroll
-    for (int jj = 0; jj < 4; ++jj) {
-      const int64_t col = w.n0 + jj * 32 + lr;
+    for (int jj = 0; jj < NJ; ++jj) {
+      const int64_t col = w.n0 + r0 + jj * 32 + lr;
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
-        const int64_t row = w.m0 + wave * 32 * NI + i * 32 + 8 * (v >> 2) + 4 * h + (v & 3);
+        const int64_t row = w.m0 + t0 + i * 32 + 8 * (v >> 2) + 4 * h + (v & 3);
         if (row < M && col < out_f) {
           if constexpr (YF32) ((float*)y)[row * out_f + col] = acc[i][jj][v];
           else ((uint16_t*)y)[row * out_f + col] = (uint16_t)f32_to_bf16_rne(acc[i][jj][v]);
@@ -443,7 +446,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     step(j + 1, 1, X1, X0);
   }
   if (j < n) step(j, 0, X0, X1);
-  ws_store<YF32>(acc, wk, wave, lane, M, out_f, grid.ltiles, y, part);
+  ws_store<YF32, 2, 4, 4>(acc, wk, wave, lane, M, out_f, grid.ltiles, y, part);
 }
 
 // ---------------------------------------------------------------------------
@@ -462,6 +465,20 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // chunk) and the decode waves' writes (2 rows x 8 atoms, one chunk of each)
 // each touch 16 different 16-byte bank groups.  The MFMA waves run the
 // one-step kernel's step four times per barrier.
+//
+// Tiles of 256, 128 or 64 tokens: MFMA wave c owns NT 32-token tiles of token
+// group c % TG and 32 TG rows of row group c / TG (256: NT 2, TG 4; 128: NT 1,
+// TG 4; 64: NT 1, TG 2).  With fewer MFMAs per tile the decode sets the pace,
+// so the 128- and 64-token tiles decode with ND = 8 waves of 16 rows.  What
+// bounds them (work-skipping copies, 14336x4096 saturated, 64 tokens, the
+// kernel alone): 29 us whole, 25.7 without the MFMAs and their operand loads,
+// 23.7 also without the decode arithmetic, 19.8 whole without the atom loads;
+// the decode's VALU is 1.0 us of a group's 2.6 us per SIMD (137 instructions
+// per atom, two decode waves), and launch, first loads and the partial tiles
+// are 9 us.  Two 64-row blocks per CU (16 waves) were no faster (M = 101: 49.8
+// against 49.8 us).  Calls against the tiled kernel these tiles replace:
+// 14336x4096 M = 101 66.7 -> 44 us, 4096x14336 66 -> 43.5, 6144x4096 40.5 ->
+// 28.5, 4096x4096 30.6 -> 23.3.
 // ---------------------------------------------------------------------------
 constexpr int kGroup = 4;                    // 64-column steps per group
 constexpr int kRowB4 = kGroup * kRowB;       // 512 bytes per tile row
@@ -469,12 +486,15 @@ constexpr int kWSlot4 = kBN * kRowB4;        // 64 KB
 
 __device__ __forceinline__ int swz4(int row, int chunk) { return chunk ^ (((chunk >> 4) & 1) << 1) ^ (row & 15); }
 
-template <bool GG, bool EXACT, bool YF32>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_ws4_kernel(
+template <bool GG, bool EXACT, bool YF32, int NT, int TG, int ND>
+__global__ __launch_bounds__(64 * (4 + ND)) __attribute__((amdgpu_waves_per_eu((4 + ND) / 4, (4 + ND) / 4)))
+void gemm_ws4_kernel(
     const uint16_t* __restrict__ x, int64_t M, const uint32_t* __restrict__ sign,
     const uint32_t* __restrict__ mant, const uint32_t* __restrict__ delta, const uint16_t* __restrict__ emax2,
     const uint8_t* __restrict__ blocks, const uint32_t* __restrict__ kp_off, const uint32_t* __restrict__ kp_ent,
     int64_t out_f, int64_t in_f, WsGrid grid, void* __restrict__ y, float* __restrict__ part) {
+  constexpr int NJ = TG;                        // 32-row W tiles per MFMA wave
+  constexpr int NR = 16 / ND;                   // rounds of a group per decode wave
   // two W slots, then 256 bytes where the plan patch lanes with no entry write
   __shared__ __attribute__((aligned(16))) uint8_t wlds[2 * kWSlot4 + 256];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -488,7 +508,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
   if (wave >= 4) {
     // ===================== decode waves =====================
-    const int pw = wave - 4;                    // 0..3
+    const int pw = wave - 4;                    // 0 .. ND - 1
     const int64_t P = in_f >> 5;                // atoms per row (a multiple of 8)
     const int a = lane & 7, rq = lane >> 3;     // atom of the group, row within a round
     using RawT = typename std::conditional<GG, RawG, Raw>::type;
@@ -497,7 +517,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     uint32_t vo_s = 0, vo_m = 0, vo_d = 0, vo_e = 0, vo_b = 0, sh = 0;
     // round 0's atom from the tile's first atom; rows past out_f read zeros
     // (buffer range check), their outputs are not stored
-    const uint32_t av = (uint32_t)((32 * pw + rq) * P) + (uint32_t)a;
+    const uint32_t av = (uint32_t)((8 * NR * pw + rq) * P) + (uint32_t)a;
     const uint32_t rstep = (uint32_t)(8 * P);   // atoms from one round's row to the next
     if constexpr (GG) {
       // P is even, so block av sits at av * 46, which is 2 (a & 1) modulo 4
@@ -544,117 +564,112 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         t.e = (uint16_t)(w.ew >> (16 * (a & 1)));
         decode_pairs(t, p);
       }
-      const int r = 32 * pw + 8 * i + rq;
+      const int r = 8 * NR * pw + 8 * i + rq;
       uint8_t* row = wlds + slot * kWSlot4 + r * kRowB4;
 #pragma unroll
       for (int c = 0; c < 4; ++c)
         *(u32x4*)(row + swz4(r, 4 * a + c) * 16) = u32x4{p[4 * c], p[4 * c + 1], p[4 * c + 2], p[4 * c + 3]};
     };
 
-    // EXACT plan: the runs of this wave's 32-row group at the 4 steps of a group
-    const int64_t G = (out_f + 31) / 32, G2 = 2 * G;
-    const int64_t gr = min(n0 / 32 + pw, G);
+    // EXACT plan: the runs of this wave's 16-row groups at the 4 steps of a
+    // group, taken as one list of their concatenated entries: entry t belongs
+    // to step u(t) = (t >= c[0]) + (t >= c[1]) + (t >= c[2]).  Lane l loads
+    // entries l, l + 64, .. (NE of them); longer lists (rare) finish behind a
+    // uniform branch.
+    constexpr int NE = ND == 4 ? 4 : 2;
+    const int64_t G2 = 2 * ((out_f + 31) / 32);
+    const int64_t gr = min(n0 / 16 + (NR / 2) * pw, G2);
     uint32_t kp_total = 0;
     if constexpr (EXACT) kp_total = kp_off[S * G2];
     const __amdgpu_buffer_rsrc_t rent = rsrc(kp_ent, (uint64_t)kp_total * 4);
     const __amdgpu_buffer_rsrc_t roff = rsrc(kp_off, ((uint64_t)S * G2 + 1) * 4);
-    const uint32_t ob = (uint32_t)(2 * gr) * 4, oe = (uint32_t)min(2 * gr + 2, G2) * 4;
-    struct Off { uint32_t beg[kGroup], end[kGroup]; };
-    struct Ent { uint32_t beg[kGroup], end[kGroup], e0[kGroup], e1[kGroup]; };
-    auto load_off = [&](int gj, Off& o) {
-      const uint32_t s0 = (uint32_t)(g0 + min(gj, ng - 1)) * kGroup;
+    // lane 2u + b: the start (b = 0) or end of step u's run
+    const uint32_t vo_o =
+        (uint32_t)(((lane >> 1) & 3) * G2 + ((lane & 1) ? min(gr + NR / 2, G2) : gr)) * 4;
+    struct Ent { uint32_t b[kGroup], c[kGroup], e[NE]; };   // run starts, ends within the list, entries
+    auto load_off = [&](int gj) {
+      return __builtin_amdgcn_raw_buffer_load_b32(
+          roff, (int)vo_o, (int)((uint32_t)(g0 + min(gj, ng - 1)) * kGroup * (uint32_t)G2 * 4u), 0);
+    };
+    auto addr_of = [&](const Ent& t, uint32_t k) {
+      return k + (k < t.c[0] ? t.b[0] : k < t.c[1] ? t.b[1] - t.c[0] : k < t.c[2] ? t.b[2] - t.c[1]
+                                                                                 : t.b[3] - t.c[2]);
+    };
+    auto load_ent = [&](uint32_t o, Ent& t) {
+      uint32_t n_ent = 0;
 #pragma unroll
       for (int u = 0; u < kGroup; ++u) {
-        o.beg[u] = __builtin_amdgcn_raw_buffer_load_b32(roff, (int)ob, (int)((s0 + u) * G2 * 4), 0);
-        o.end[u] = __builtin_amdgcn_raw_buffer_load_b32(roff, (int)oe, (int)((s0 + u) * G2 * 4), 0);
+        t.b[u] = __builtin_amdgcn_readlane(o, 2 * u);
+        n_ent += __builtin_amdgcn_readlane(o, 2 * u + 1) - t.b[u];
+        t.c[u] = n_ent;
       }
-    };
-    auto load_ent = [&](const Off& o, Ent& e) {
 #pragma unroll
-      for (int u = 0; u < kGroup; ++u) {
-        e.beg[u] = __builtin_amdgcn_readfirstlane(o.beg[u]);
-        e.end[u] = __builtin_amdgcn_readfirstlane(o.end[u]);
-        e.e0[u] = __builtin_amdgcn_raw_buffer_load_b32(rent, (int)((e.beg[u] + lane) * 4), 0, 0);
-        e.e1[u] = __builtin_amdgcn_raw_buffer_load_b32(rent, (int)((e.beg[u] + lane + 64) * 4), 0, 0);
-      }
+      for (int k = 0; k < NE; ++k)
+        t.e[k] = __builtin_amdgcn_raw_buffer_load_b32(rent, (int)(addr_of(t, lane + 64 * k) * 4), 0, 0);
     };
-    // entry -> its bf16 in the group tile (step u of the group); a lane past
-    // the run writes its own word of the spare area instead (no exec-mask
-    // branch); the empty asm makes the compiler wait for the entry's load
-    // there
-    auto patch_one = [&](uint32_t e, int slot, int u, bool live) {
+    // entry -> its bf16 in the group tile; a lane past the list writes its
+    // own word of the spare area instead (no exec-mask branch); the empty asm
+    // makes the compiler wait for the entry's load there
+    auto patch_one = [&](const Ent& t, uint32_t k, uint32_t e, int slot, bool live) {
+      const int u = (k >= t.c[0]) + (k >= t.c[1]) + (k >= t.c[2]);
       const int rr = (int)(e >> 22) & (kBN - 1), c = (int)(e >> 16) & 63;
       const uint32_t dst =
           (uint32_t)(slot * kWSlot4 + rr * kRowB4 + swz4(rr, 8 * u + chunk_of(c)) * 16 + pos_of(c) * 2);
       __asm__ volatile("" : "+v"(e));
       *(uint16_t*)(wlds + (live ? dst : (uint32_t)(2 * kWSlot4 + lane * 4))) = (uint16_t)(e & 0xFFFFu);
     };
-    // the first 64 entries of each step's run; runs longer than 64 (rare)
-    // behind one uniform branch
-    auto patch = [&](const Ent& e, int slot) {
-      uint32_t longest = 0;
+    auto patch = [&](const Ent& t, int slot) {
 #pragma unroll
-      for (int u = 0; u < kGroup; ++u) {
-        patch_one(e.e0[u], slot, u, e.beg[u] + lane < e.end[u]);
-        longest = max(longest, e.end[u] - e.beg[u]);
-      }
-      if (longest > 64) {
-#pragma unroll
-        for (int u = 0; u < kGroup; ++u) {
-          if (e.beg[u] + lane + 64 < e.end[u]) patch_one(e.e1[u], slot, u, true);
-          for (uint32_t k = e.beg[u] + 128 + lane; k < e.end[u]; k += 64)   // dense runs
-            patch_one(kp_ent[k], slot, u, true);
-        }
-      }
+      for (int k = 0; k < NE; ++k) patch_one(t, lane + 64 * k, t.e[k], slot, lane + 64 * k < t.c[3]);
+      if (t.c[3] > 64 * NE)
+        for (uint32_t k = 64 * NE + lane; k < t.c[3]; k += 64)
+          patch_one(t, k, kp_ent[min(addr_of(t, k), kp_total - 1)], slot, true);
     };
 
-    RawT R[4];
-    Off O{};
-    Ent E{};
+    RawT R[NR];
+    uint32_t O = 0;
+    Ent E[2] = {};
     // prologue: group 0's plan offsets and entries and group 1's offsets,
-    // group 0's atoms; group 0 decoded round by round, each round's registers
-    // refilled with group 1's atoms; then group 1's entries and group 2's
-    // offsets.  The loads in flight at the loop entry are then 4 rounds of
-    // atoms, entries, offsets, as at the end of every iteration.
-    if constexpr (EXACT) load_off(0, O);
+    // group 0's atoms; group 1's entries and group 2's offsets; group 0 decoded
+    // round by round, each round's registers refilled with group 1's atoms.
+    // The plan is requested ahead of the atoms everywhere (waits are in request
+    // order), so waiting for a group's entries leaves the atoms requested
+    // after them in flight.  One group of atoms ahead is enough: with two the
+    // 8-decode-wave tiles were 1.3 us slower (14336x4096 M = 64: 39.9 against
+    // 38.6), the second group only lengthening the prologue's burst.
+    if constexpr (EXACT) O = load_off(0);
     __builtin_amdgcn_sched_barrier(0);
-    if constexpr (EXACT) { load_ent(O, E); load_off(1, O); }
+    if constexpr (EXACT) { load_ent(O, E[0]); O = load_off(1); }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) load_round(0, i, R[i]);
+    for (int i = 0; i < NR; ++i) load_round(0, i, R[i]);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (EXACT) { load_ent(O, E[1]); O = load_off(2); }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < NR; ++i) {
       store_round(R[i], i, 0);
       __builtin_amdgcn_sched_barrier(0);
       load_round(1, i, R[i]);
       __builtin_amdgcn_sched_barrier(0);
     }
-    if constexpr (EXACT) {
-      patch(E, 0);
-      __builtin_amdgcn_sched_barrier(0);
-      load_ent(O, E);
-      load_off(2, O);
-    }
+    if constexpr (EXACT) patch(E[0], 0);
     __builtin_amdgcn_sched_barrier(0);
     __syncthreads();
 
-    // iteration j: group j + 1 decoded into slot (j + 1) & 1, round by round,
-    // each round's registers refilled with group j + 2's atoms; its plan
-    // entries patched, then group j + 2's entries and group j + 3's offsets
+    // iteration j: group j + 2's entries and group j + 3's offsets requested;
+    // group j + 1 decoded into slot (j + 1) & 1, round by round, each round's
+    // registers refilled with group j + 2's atoms; its entries patched
     auto iter = [&](int j, int slot) {
+      if constexpr (EXACT) { load_ent(O, E[slot ^ 1]); O = load_off(j + 3); }
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
+      for (int i = 0; i < NR; ++i) {
         store_round(R[i], i, slot);
         __builtin_amdgcn_sched_barrier(0);
         load_round(j + 2, i, R[i]);
         __builtin_amdgcn_sched_barrier(0);
       }
-      if constexpr (EXACT) {
-        patch(E, slot);
-        __builtin_amdgcn_sched_barrier(0);
-        load_ent(O, E);
-        load_off(j + 3, O);
-      }
+      if constexpr (EXACT) patch(E[slot], slot);
       __builtin_amdgcn_sched_barrier(0);
       __syncthreads();
     };
@@ -673,15 +688,17 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int s0 = g0 * kGroup;
   const int64_t S64 = S;
   const __amdgpu_buffer_rsrc_t rx_ = rsrc(x + m0 * in_f, (uint64_t)(((M + 31) / 32) * 32 - m0) * (uint64_t)in_f * 2);
-  const uint32_t vx0 = (uint32_t)(2 * wave * S64 * 4096 + lane * 16);
-  const uint32_t vx1 = vx0 + (uint32_t)(S64 * 4096);
-  auto load_x = [&](int jx, bf16x8_t (&X)[2][4]) {
+  const int tw = wave % TG, jw = wave / TG;   // token group and W row group of this wave
+  uint32_t vx[NT];
+#pragma unroll
+  for (int i = 0; i < NT; ++i) vx[i] = (uint32_t)((NT * tw + i) * S64 * 4096 + lane * 16);
+  auto load_x = [&](int jx, bf16x8_t (&X)[NT][4]) {
     const uint32_t ks = (uint32_t)(s0 + min(jx, n - 1)) * 4096;
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < NT; ++i)
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rx_, (int)((i ? vx1 : vx0) + q * 1024), (int)ks, 0);
+        const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rx_, (int)(vx[i] + q * 1024), (int)ks, 0);
         X[i][q] = __builtin_bit_cast(bf16x8_t, v);
       }
   };
@@ -691,53 +708,107 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   // the slot is bit 16 of the address and jj an immediate offset.
   uint32_t wo[4];
 #pragma unroll
-  for (int q = 0; q < 4; ++q) wo[q] = (uint32_t)(lr * kRowB4 + (((4 * h + q) ^ (lr & 15)) * 16));
-  auto load_w = [&](int q, int u, int slot, bf16x8_t (&wb)[4]) {
+  for (int q = 0; q < 4; ++q)
+    wo[q] = (uint32_t)((jw * NJ * 32 + lr) * kRowB4 + (((4 * h + q) ^ (lr & 15)) * 16));
+  auto load_w = [&](int q, int u, int slot, bf16x8_t (&wb)[NJ]) {
     const uint32_t ku = (uint32_t)(((8 * u) ^ ((u >> 1) << 1)) * 16) | ((uint32_t)slot << 16);
     const uint32_t o = wo[q] ^ ku;
 #pragma unroll
-    for (int jj = 0; jj < 4; ++jj) wb[jj] = *(const bf16x8_t*)(wlds + o + jj * 32 * kRowB4);
+    for (int jj = 0; jj < NJ; ++jj) wb[jj] = *(const bf16x8_t*)(wlds + o + jj * 32 * kRowB4);
   };
-  f32x16 acc[2][4];
+  f32x16 acc[NT][NJ];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < NT; ++i)
 #pragma unroll
-    for (int jj = 0; jj < 4; ++jj)
+    for (int jj = 0; jj < NJ; ++jj)
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[i][jj][v] = 0.f;
-  auto mfma = [&](int t, const bf16x8_t (&X)[2][4], int q, const bf16x8_t (&wb)[4]) {
-    const int i = t >> 2, jj = t & 3;
+  constexpr int NM = NT * NJ;                 // MFMAs per k-quarter
+  if constexpr (NT == 1) {
+    // Few MFMAs per k-quarter: a quarter's operands are requested into the
+    // registers of the quarter just multiplied, WD steps (W, from LDS) and XD
+    // steps (x) ahead, so an LDS read has at least three quarters' MFMAs to
+    // arrive.  The group's last WD steps request the next group's operands:
+    // the barrier comes before them, when all of this group's are in
+    // registers, which also frees the slot for the decode waves early.
+    constexpr int WD = NJ == 4 ? 1 : 2, XD = WD;
+    bf16x8_t X[XD][4], W[WD][4][NJ];
+    auto load_xq = [&](int jx, int q, bf16x8_t& d) {
+      const uint32_t ks = (uint32_t)(s0 + min(jx, n - 1)) * 4096;
+      const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rx_, (int)(vx[0] + q * 1024), (int)ks, 0);
+      d = __builtin_bit_cast(bf16x8_t, v);
+    };
+    auto group = [&](int jg, int slot) {
+#pragma unroll
+      for (int u = 0; u < kGroup; ++u) {
+        if (u == kGroup - WD) {
+          __builtin_amdgcn_sched_barrier(0);
+          __syncthreads();
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        const int nu = (u + WD) % kGroup, ns = u + WD >= kGroup ? slot ^ 1 : slot;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+#pragma unroll
+          for (int jj = 0; jj < NJ; ++jj)
+            acc[0][jj] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(X[u % XD][q], W[u % WD][q][jj], acc[0][jj], 0, 0, 0);
+          load_xq(4 * jg + u + XD, q, X[u % XD][q]);
+          load_w(q, nu, ns, W[u % WD][q]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    };
+#pragma unroll
+    for (int u = 0; u < XD; ++u)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) load_xq(u, q, X[u][q]);
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < WD; ++u)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) load_w(q, u, 0, W[u][q]);
+    __builtin_amdgcn_sched_barrier(0);
+    int jg = 0;
+    for (; jg + 1 < ng; jg += 2) {
+      group(jg, 0);
+      group(jg + 1, 1);
+    }
+    if (jg < ng) group(jg, 0);
+  } else {
+  auto mfma = [&](int t, const bf16x8_t (&X)[NT][4], int q, const bf16x8_t (&wb)[NJ]) {
+    const int i = t / NJ, jj = t % NJ;
     acc[i][jj] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(X[i][q], wb[jj], acc[i][jj], 0, 0, 0);
   };
 #define BF16X_SG(mask, cnt) __builtin_amdgcn_sched_group_barrier(mask, cnt, 0)
-  bf16x8_t X0[2][4], X1[2][4], W0[4], W1[4];
+#define BF16X_SG(mask, cnt) __builtin_amdgcn_sched_group_barrier(mask, cnt, 0)
+  bf16x8_t X0[NT][4], X1[NT][4], W0[NJ], W1[NJ];
   // step u of the group in `slot` (block step jx) with x in X; x of step
   // jx + 1 requested into Xn first.  The last quarter's second half reads
   // the next step's quarter-0 W operands: after the group's barrier from the
   // other slot at u == 3, from the same slot otherwise.
-  auto step = [&](int jx, int u, int slot, const bf16x8_t (&X)[2][4], bf16x8_t (&Xn)[2][4]) {
+  auto step = [&](int jx, int u, int slot, const bf16x8_t (&X)[NT][4], bf16x8_t (&Xn)[NT][4]) {
     load_x(jx + 1, Xn);
     load_w(1, u, slot, W1);
 #pragma unroll
-    for (int t = 0; t < 8; ++t) mfma(t, X, 0, W0);
-    BF16X_SG(0x020, 8);
-    BF16X_SG(0x100, 4);
-    BF16X_SG(0x008, 8);
+    for (int t = 0; t < NM; ++t) mfma(t, X, 0, W0);
+    BF16X_SG(0x020, 4 * NT);
+    BF16X_SG(0x100, NJ);
+    BF16X_SG(0x008, NM);
     __builtin_amdgcn_sched_barrier(0);
     load_w(2, u, slot, W0);
 #pragma unroll
-    for (int t = 0; t < 8; ++t) mfma(t, X, 1, W1);
-    BF16X_SG(0x100, 4);
-    BF16X_SG(0x008, 8);
+    for (int t = 0; t < NM; ++t) mfma(t, X, 1, W1);
+    BF16X_SG(0x100, NJ);
+    BF16X_SG(0x008, NM);
     __builtin_amdgcn_sched_barrier(0);
     load_w(3, u, slot, W1);
 #pragma unroll
-    for (int t = 0; t < 8; ++t) mfma(t, X, 2, W0);
-    BF16X_SG(0x100, 4);
-    BF16X_SG(0x008, 8);
+    for (int t = 0; t < NM; ++t) mfma(t, X, 2, W0);
+    BF16X_SG(0x100, NJ);
+    BF16X_SG(0x008, NM);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int t = 0; t < 4; ++t) mfma(t, X, 3, W1);
+    for (int t = 0; t < NM / 2; ++t) mfma(t, X, 3, W1);
     __builtin_amdgcn_sched_barrier(0);
     if (u == kGroup - 1) {
       __syncthreads();
@@ -746,9 +817,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       load_w(0, u + 1, slot, W0);
     }
 #pragma unroll
-    for (int t = 4; t < 8; ++t) mfma(t, X, 3, W1);
-    BF16X_SG(0x100, 4);
-    BF16X_SG(0x008, 4);
+    for (int t = NM / 2; t < NM; ++t) mfma(t, X, 3, W1);
+    BF16X_SG(0x100, NJ);
+    BF16X_SG(0x008, NM - NM / 2);
     __builtin_amdgcn_sched_barrier(0);
   };
 #undef BF16X_SG
@@ -767,7 +838,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     group(jg + 1, 1);
   }
   if (jg < ng) group(jg, 0);
-  ws_store<YF32>(acc, wk, wave, lane, M, out_f, grid.ltiles, y, part);
+  }
+  ws_store<YF32, NT, TG, NJ>(acc, wk, wave, lane, M, out_f, grid.ltiles, y, part);
 }
 
 // x [M, K] -> operand order: 32-row tile T, step s (64 columns), k-quarter q
@@ -870,6 +942,25 @@ int64_t ws_resident() {
   return cus;
 }
 
+// Token rows per tile of the grouped kernel.  A tile of 64 tokens decodes its W
+// rows in about the time of a 128-token tile (the decode sets the pace), a
+// 256-token tile in a third more, so a tile covers all tokens up to 256 unless
+// two smaller token tiles still leave every CU at most one block before K is
+// split (C / 4: their shorter K ranges and smaller partials then win).
+// Measured, exact, 64 / 128 / 256-token tiles (us): 14336x4096 M = 64 38.6 /
+// 42.1 / 48.7, M = 128 52.8 / 45.3 / 51.1, M = 191 74.9 / 60.7 / 54.3;
+// 4096x4096 (32 row tiles) M = 64 22.6 / 24.1 / 28.8, M = 128 23.8 / 24.9 /
+// 29.5, M = 191 30.1 / 27.3 / 30.7.
+int64_t ws_tile_rows(int64_t M, int64_t nt, int64_t C) {
+  const int64_t t = tuning(BF16X_TUNE_GEMM_WS_BM);
+  if (t == 64 || t == 128 || t == 256) return t;
+  for (int64_t bm = 64; bm < 256; bm *= 2) {
+    const int64_t mt = (M + bm - 1) / bm;
+    if (mt == 1 || (mt == 2 && mt * nt <= C / 4)) return bm;
+  }
+  return 256;
+}
+
 // Tiles run whole-K in full rounds of resident blocks; the f tiles of the
 // last, partial round (all tiles when there are fewer than one round) are
 // split into s = min(resident / f, 16) K ranges of at least one group (four
@@ -882,13 +973,14 @@ int64_t ws_resident() {
 WsShape ws_shape(int64_t M, int64_t out_f, int64_t in_f) {
   WsShape w;
   w.grouped = ws_grouped(in_f);
-  const int64_t bm = kBM;
-  const int64_t mt = (M + bm - 1) / bm, nt = (out_f + kBN - 1) / kBN;
+  const int64_t forced_c = tuning(BF16X_TUNE_GEMM_WS_RESIDENT);
+  const int64_t C = forced_c > 0 ? forced_c : ws_resident();
+  const int64_t nt = (out_f + kBN - 1) / kBN;
+  const int64_t bm = w.grouped ? ws_tile_rows(M, nt, C) : kBM;
+  const int64_t mt = (M + bm - 1) / bm;
   const int64_t S = in_f / kStep, tiles = mt * nt;
   const int64_t units = w.grouped ? S / kGroup : S;
   const int64_t max_split = std::max<int64_t>(1, std::min<int64_t>(16, w.grouped ? units : units / 4));
-  const int64_t forced_c = tuning(BF16X_TUNE_GEMM_WS_RESIDENT);
-  const int64_t C = forced_c > 0 ? forced_c : ws_resident();
   int64_t f = tiles % C, s = f ? std::min<int64_t>(C / f, max_split) : 1;
   const int64_t forced = tuning(BF16X_TUNE_GEMM_WS_SPLIT);
   if (forced > 0) {
@@ -942,14 +1034,17 @@ int bf16x_gemm_ws_launch(const uint16_t* x, int64_t M, const uint32_t* s, const 
   const uint16_t* xo = (const uint16_t*)workspace;
   float* part = (float*)((uint8_t*)workspace + xop);
   const dim3 grid((unsigned)w.grid);
+#define BF16X_WS4(GG_, EX_, YF_, NT_, TG_, ND_)                                                                   \
+  hipLaunchKernelGGL((gemm_ws4_kernel<GG_, EX_, YF_, NT_, TG_, ND_>), grid, dim3(64 * (4 + ND_)), 0, st, xo, M, s, m, \
+                     d, e, blocks, kp_off, kp_ent, out_f, in_f, w.g, y, part)
 #define BF16X_WS1(GG_, EX_, YF_)                                                                                   \
   do {                                                                                                           \
-    if (w.grouped)                                                                                               \
-      hipLaunchKernelGGL((gemm_ws4_kernel<GG_, EX_, YF_>), grid, dim3(512), 0, st, xo, M, s, m, d, e, blocks,       \
-                         kp_off, kp_ent, out_f, in_f, w.g, y, part);                                              \
-    else                                                                                                         \
+    if (!w.grouped)                                                                                              \
       hipLaunchKernelGGL((gemm_ws_kernel<GG_, EX_, YF_>), grid, dim3(512), 0, st, xo, M, s, m, d, e, blocks,        \
                          kp_off, kp_ent, out_f, in_f, w.g, y, part);                                              \
+    else if (w.g.bm == 64) BF16X_WS4(GG_, EX_, YF_, 1, 2, 8);                                                     \
+    else if (w.g.bm == 128) BF16X_WS4(GG_, EX_, YF_, 1, 4, 8);                                                    \
+    else BF16X_WS4(GG_, EX_, YF_, 2, 4, 4);                                                                       \
   } while (0)
 #define BF16X_WS(GG_)                                        \
   do {                                                       \
@@ -965,6 +1060,7 @@ int bf16x_gemm_ws_launch(const uint16_t* x, int64_t M, const uint32_t* s, const 
   else BF16X_WS(false);
 #undef BF16X_WS
 #undef BF16X_WS1
+#undef BF16X_WS4
   if (w.nsplit > 1) {
     const int64_t count = (int64_t)w.g.ltiles * ((int64_t)w.g.bm * kBN);
     const int64_t blocks_r = std::min<int64_t>((count / 4 + 255) / 256, 4096);

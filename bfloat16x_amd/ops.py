@@ -314,14 +314,21 @@ GEMM_ROWS_IN_F = (2048, 4096)
 # Activation rows for which bf16x_gemm runs the chunked few-row kernel
 # (bf16x_gemm_chunks: in_f % 256 == 0), for weights of at most
 # GEMM_CHUNKS_MAX_IN_F columns, except above 32 rows when a CU has 16 rows or
-# fewer (each CU then reads more x than weight).  Measured, exact, weights
+# fewer (each CU then reads more x than weight), or when the weight has
+# GEMM_CHUNKS_LARGE elements or more (three quarters of that above 47 rows):
+# there bf16x_gemm's wave-specialised kernel, whose fixed cost is larger and
+# whose cost per weight is smaller, is faster.  Measured, exact, weights
 # rotated through HBM, chunked against the 16x16x32 few-row kernel (us):
 # 14336x4096 M = 24 / 32 / 48 / 64: 29.0 / 30.2 / 36.8 / 38.7 against 32.0 /
 # 32.0 / 43.0 / 44.3; 4096x4096 M = 24 / 32: 16.4 / 17.5 against 19.9 / 19.6,
-# M = 64: 22.6 against 20.8; 4096x14336 M = 32: 44.9 against 33.8.
+# M = 64: 22.6 against 20.8; 4096x14336 M = 32: 44.9 against 33.8.  Against
+# the wave-specialised kernel: 28672x4096 M = 24 / 33 / 64 59.9 / 68.7 / 77.9
+# against 57.2 / 59.1 / 60.6; 14336x4096 M = 33 / 48 / 64 36.0 / 38.4 / 40.5
+# against 38.7 / 38.3 / 38.6; 6144x4096 M = 64 25.1 against 25.1.
 GEMM_CHUNKS_MIN = 17
 GEMM_CHUNKS_MAX = 64
 GEMM_CHUNKS_MAX_IN_F = 8192
+GEMM_CHUNKS_LARGE = 1 << 26
 
 
 def _cus(dev) -> int:
@@ -331,7 +338,10 @@ def _cus(dev) -> int:
 def _use_chunks(M: int, out_f: int, in_f: int, dev) -> bool:
     if not (GEMM_CHUNKS_MIN <= M <= GEMM_CHUNKS_MAX) or in_f % 256 or in_f > GEMM_CHUNKS_MAX_IN_F:
         return False
-    return M <= 32 or -(-out_f // _cus(dev)) > 16
+    if M <= 32:
+        return True
+    large = GEMM_CHUNKS_LARGE if M < 48 else GEMM_CHUNKS_LARGE * 3 // 4
+    return out_f * in_f < large and -(-out_f // _cus(dev)) > 16
 # One bf16 activation row goes to the GEMV (bf16x_gemv), which streams the
 # weight faster than any GEMM kernel at one row (14336x4096: 19.4 against
 # 24.2 us for the row-streaming GEMM).

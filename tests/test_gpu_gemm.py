@@ -244,3 +244,62 @@ def test_gemm_ws_split_sum_is_deterministic(bx, tune, split):
                                ys[0].view(torch.int32 if dt == torch.float32 else torch.int16))
     mx, med = dc.rel_err(ys[0].float().cpu().numpy(), dc.gemm_ref(_np(d), x.float().cpu().numpy(), saturated=False))
     assert mx <= 1e-2 and med <= 2e-3, (mx, med)
+
+
+# Token tiles of the grouped kernel: one token, a tile less one / whole / plus
+# one token, two tiles, ragged out_f; K in one range, three, and the dispatch's
+# own; "spread" exponents put most elements in the plan (lists longer than the
+# entries a decode wave reads ahead).  Against float64 of the same weight:
+# outputs are fp32 sums of in_f exact products rounded once to bf16.
+@pytest.mark.parametrize("bm", [64, 128, 256])
+@pytest.mark.parametrize("M", [1, 63, 64, 65, 128, 129, 257])
+@pytest.mark.parametrize("kind,out_f,in_f,split", [("bench", 300, 1024, -1), ("bench", 130, 4096, 3),
+                                                   ("bench", 256, 256, 1), ("spread", 200, 768, -1)])
+def test_gemm_ws_token_tiles(bx, tune, bm, M, kind, out_f, in_f, split):
+    tune(gemm_ws_bm=bm, gemm_ws_split=split, gemm_skinny2_max=0, gemm_skinny_max=0, gemm_ws_min_rows=1)
+    if kind == "bench":
+        bits = dc.bench_weight_bits(out_f, in_f, seed=M)
+    else:
+        rng = np.random.default_rng(M)
+        bits = ((rng.integers(0, 2, (out_f, in_f)) << 15) | (rng.integers(100, 128, (out_f, in_f)) << 7)
+                | rng.integers(0, 128, (out_f, in_f))).astype(np.uint16)
+    w = bits_tensor(bits)
+    d = bx.bf16x_quantize(w)
+    g = to_dev(d)
+    plan = bx.build_plan_host(d, device=DEV)
+    sat = bits_tensor(dc.decode_saturated(_np(d)).reshape(out_f, in_f))
+    x = torch.randn(M, in_f, generator=torch.Generator().manual_seed(M)).to(torch.bfloat16)
+    L = bx._lib.lib()
+    kp = plan.kplan()
+    for p, wr in ((plan, w), (None, sat)):
+        ref = (x.to(DEV).double() @ wr.to(DEV).double().t().contiguous()).cpu().numpy()
+        ws = torch.empty(int(L.bf16x_gemm_workspace(M, out_f, in_f)) // 4 + 4, dtype=torch.float32, device=DEV)
+        for dt, code in ((torch.bfloat16, bx._lib.BF16), (torch.float32, bx._lib.F32)):
+            y = torch.empty(M, out_f, dtype=dt, device=DEV)
+            xd = x.to(DEV)
+            st = L.bf16x_gemm(xd.data_ptr(), bx._lib.BF16, M, g["sign_packed"].data_ptr(), g["sign_packed"].numel(),
+                              g["mant_packed"].data_ptr(), g["mant_packed"].numel(), g["delta_packed"].data_ptr(),
+                              g["delta_packed"].numel(), g["emax"].data_ptr(), g["emax"].numel(),
+                              kp[0].data_ptr() if p is not None else None,
+                              kp[1].data_ptr() if p is not None else None, out_f, in_f, 16,
+                              bx._lib.EXACT if p is not None else bx._lib.SATURATED, y.data_ptr(), code,
+                              ws.data_ptr(), ws.numel() * 4, bx._lib.stream_of(xd.device))
+            assert st == 0
+            check_tol(y.double().cpu().numpy(), ref)
+
+
+# The dispatch's own choice on both sides of its lines: 64 / 65 rows, 32 / 33
+# rows of a weight of 2^25 elements, in_f not a multiple of 256 (no four-step
+# groups)
+@pytest.mark.parametrize("M,out_f,in_f", [(64, 640, 1024), (65, 640, 1024), (191, 640, 1024), (65, 640, 1088),
+                                          (32, 2048, 16384), (33, 2048, 16384), (64, 2048, 16384),
+                                          (48, 12288, 4096), (33, 16384, 4096)])
+def test_gemm_dispatch_lines(bx, M, out_f, in_f):
+    g = torch.Generator(device=DEV).manual_seed(M)
+    w = (torch.randn(out_f, in_f, generator=g, device=DEV) * 0.02).to(torch.bfloat16)
+    w[:, ::97] *= 30
+    d = bx.bf16x_quantize(w)
+    plan = bx.build_plan_host(d, device=DEV)
+    x = torch.randn(M, in_f, generator=g, device=DEV).to(torch.bfloat16)
+    y = bx.bf16x_gemm(x, d["sign_packed"], d["mant_packed"], d["delta_packed"], d["emax"], out_f, in_f, plan=plan)
+    check_tol(y.double().cpu().numpy(), (x.double() @ w.double().t().contiguous()).cpu().numpy())

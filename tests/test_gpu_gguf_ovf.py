@@ -117,3 +117,23 @@ def test_tampered_table_refused(g):
     blob[off + 3] ^= 0x80
     with pytest.raises(_lib.Bf16xError):
         g.device_ovf(bytes(blob), packed, DEV)
+
+
+# Token tiles of the fused GEMM (64, 128 and 256 tokens), one token either
+# side, lossless ("dense": lists longer than a decode wave reads ahead) and
+# near-lossless
+@pytest.mark.parametrize("kind,shape", [("dense", (300, 1024)), ("selftest", (130, 256))])
+@pytest.mark.parametrize("M", [2, 64, 65, 128, 129])
+def test_gemm_fused_token_tiles(g, tune, kind, shape, M):
+    w = weights(kind, shape, 10)
+    wb = go.bf16_bits_to_fp32(go.fp32_to_bf16_bits(w)).astype(np.float64).reshape(shape)
+    packed = g.quantize_blocks(w)
+    wnl = go.dequantize_blocks(packed).astype(np.float64).reshape(shape)
+    t = g.device_ovf(g.pack_ovf(w), packed, DEV)
+    blocks = g.device_blocks(packed, DEV)
+    xm = torch.randn(M, shape[1], generator=torch.Generator().manual_seed(M)).to(torch.bfloat16)
+    for bm in (64, 128, 256):
+        tune(gemm_ws_bm=bm)
+        for ovf, ref in ((t, wb), (None, wnl)):
+            y = g.gguf_gemm_fused(xm.to(DEV), blocks, *shape, out_dtype=torch.float32, ovf=ovf)
+            check_tol(y.cpu().numpy(), xm.double().numpy() @ ref.T)
