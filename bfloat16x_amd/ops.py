@@ -378,6 +378,28 @@ def _gemm_launch(x2, s, m, d, e, out_f, in_f, plan, y, y_dtype, sub=16):
     _lib.check(st, "bf16x_gemm")
 
 
+def _gemm_terms(x2, s, m, d, e, out_f, in_f, plan, sub):
+    """x2 (fp16 or fp32) . W^T in x2's dtype: x = hi + lo as two bf16 terms
+    (exact for fp16, 16 significant bits for fp32), the products in fp32.
+    The terms are the 2 M rows of one launch, which decodes W once for both;
+    where 2 M rows pass the kernels' 32-bit offsets, one launch each."""
+    L = _lib.lib()
+    M, dev, st = x2.shape[0], x2.device, _lib.stream_of(x2.device)
+    terms = torch.empty(2, M, in_f, dtype=torch.bfloat16, device=dev)
+    _lib.check(L.bf16x_split_terms(x2.data_ptr(), _X_DTYPES[x2.dtype], x2.numel(), terms[0].data_ptr(),
+                                   terms[1].data_ptr(), st), "bf16x_split_terms")
+    parts = torch.empty(2, M, out_f, dtype=torch.float32, device=dev)
+    if 2 * M * in_f * 2 < 0xFFFFFFFF:
+        _gemm_launch(terms.view(2 * M, in_f), s, m, d, e, out_f, in_f, plan, parts.view(2 * M, out_f), _lib.F32, sub)
+    else:
+        for k in range(2):
+            _gemm_launch(terms[k], s, m, d, e, out_f, in_f, plan, parts[k], _lib.F32, sub)
+    y = torch.empty(M, out_f, dtype=x2.dtype, device=dev)
+    _lib.check(L.bf16x_add_terms(parts[0].data_ptr(), parts[1].data_ptr(), y.numel(), y.data_ptr(),
+                                 _X_DTYPES[y.dtype], st), "bf16x_add_terms")
+    return y
+
+
 # From this many activation rows on, bf16x_gemm decodes W once at HBM speed
 # and runs the product as a plain library GEMM (hipBLASLt through
 # F.linear): the decode is amortised over the rows and the library GEMM runs
@@ -412,8 +434,8 @@ def bf16x_gemm(x, sign, mant, delta, emax, out_f, in_f, plan: Bf16xPlan | None =
     GEMM_CHUNKS_MIN to GEMM_CHUNKS_MAX rows (see _use_chunks), else
     bf16x_gemm in the C ABI; one bf16 row the fused GEMV, bf16x_gemv);
     bf16 activations run one bf16 MFMA pass, fp16/fp32 activations are split
-    as x = hi + lo (two bf16 tensors, exact for fp16, 16 mantissa bits for
-    fp32) accumulated over two passes in fp32.
+    as x = hi + lo (two bf16 terms, exact for fp16, 16 mantissa bits for
+    fp32), the rows of both in one launch, and added in fp32.
     path "decode": W decoded into a temporary by the HIP decoder, then
     F.linear on the same device (fp32 for fp16/fp32 activations).
     path "auto": "decode" from GEMM_DECODE_MIN_ROWS rows on (_TALL / _WIDE for
@@ -447,14 +469,7 @@ def bf16x_gemm(x, sign, mant, delta, emax, out_f, in_f, plan: Bf16xPlan | None =
         y = torch.empty(x2.shape[0], out_f, dtype=torch.bfloat16, device=xx.device)
         _gemm_launch(x2.contiguous(), s, m, d, e, out_f, in_f, plan, y, _lib.BF16, sub)
     else:
-        xf = x2.float()
-        hi = xf.to(torch.bfloat16)
-        lo = (xf - hi.float()).to(torch.bfloat16)
-        y = torch.empty(x2.shape[0], out_f, dtype=torch.float32, device=xx.device)
-        y2 = torch.empty_like(y)
-        _gemm_launch(hi.contiguous(), s, m, d, e, out_f, in_f, plan, y, _lib.F32, sub)
-        _gemm_launch(lo.contiguous(), s, m, d, e, out_f, in_f, plan, y2, _lib.F32, sub)
-        y = (y + y2).to(xx.dtype)
+        y = _gemm_terms(x2, s, m, d, e, out_f, in_f, plan, sub)
     return y.reshape(*lead, out_f)
 
 

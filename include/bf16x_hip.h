@@ -280,6 +280,13 @@ int bf16x_gemm_chunks(const void* x, int32_t x_dtype, int64_t M,
                       int64_t out_f, int64_t in_f, int32_t sub, int32_t mode,
                       void* y, int32_t y_dtype, bf16x_stream_t stream);
 
+/* fp16 / fp32 activations as two bf16 terms x = hi + lo (hi = bf16(x), lo =
+ * bf16(x - hi)) for the products above, and the sum of two fp32 results in
+ * x's type.  x_dtype / y_dtype: BF16X_F16 or BF16X_F32.  n elements, all
+ * pointers dev, each aligned to its element. */
+int bf16x_split_terms(const void* x, int32_t x_dtype, int64_t n, uint16_t* hi, uint16_t* lo, bf16x_stream_t stream);
+int bf16x_add_terms(const float* a, const float* b, int64_t n, void* y, int32_t y_dtype, bf16x_stream_t stream);
+
 /* ========================================================================
  * GGUF half-block variant (bf16x_gguf_block.py, GGML_TYPE_BF16X): blocks of
  * 32 row-major weights, 46 bytes = [emax[2] | sign[4] | mant[28] |
