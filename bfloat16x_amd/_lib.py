@@ -145,6 +145,24 @@ def lib() -> ctypes.CDLL:
     return _LIB
 
 
+_HOST = None
+
+
+def host():
+    """The native host path of the hot wrappers (_host.so, csrc/host_ext.cpp);
+    raises if it was not built."""
+    global _HOST
+    if _HOST is None:
+        lib()
+        try:
+            from . import _host
+        except ImportError as e:
+            raise RuntimeError(f"{os.path.join(HERE, '_host.so')} is missing or does not load ({e}): build it with "
+                               "`python -m bfloat16x_amd.build`") from e
+        _HOST = _host
+    return _HOST
+
+
 def status_string(status: int) -> str:
     try:
         return lib().bf16x_status_string(int(status)).decode()
@@ -164,7 +182,8 @@ def ptr(t) -> int | None:
 
 def stream_of(device: torch.device):
     """Raw hipStream_t of torch's current stream on `device`."""
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    index = device.index
+    return host().stream(torch.cuda.current_device() if index is None else index)
 
 
 def version() -> str:

@@ -1,10 +1,11 @@
-"""Build libbf16x_hip.so in-tree with hipcc for gfx950.
+"""Build libbf16x_hip.so (hipcc, gfx950) and _host.so in-tree.
 
     python -m bfloat16x_amd.build [-v]
 
 Every HIP source is compiled for gfx950 with packed-fp32 instruction
 selection disabled, host C++ sources with the same driver, and the objects
-are linked into bfloat16x_amd/libbf16x_hip.so.  Objects go to _build/
+are linked into bfloat16x_amd/libbf16x_hip.so.  csrc/host_ext.cpp, the CPython
+module over torch's C++ API, is compiled with g++ into bfloat16x_amd/_host.so.  Objects go to _build/
 (ignored by git).
 """
 from __future__ import annotations
@@ -15,11 +16,14 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "libbf16x_hip.so")
+HOST_SRC = os.path.join(CSRC, "host_ext.cpp")
+HOST_OUT = os.path.join(HERE, "_host.so")
 BUILD_DIR = os.path.join(ROOT, "_build", "bf16x_hip")
 ARCH = "gfx950"
 
@@ -55,9 +59,31 @@ def _compile(src: str, verbose: bool) -> str:
     return obj
 
 
+def _build_host(verbose: bool) -> None:
+    """_host.so: links libbf16x_hip.so beside it and torch's libraries (which
+    are loaded already when it is imported)."""
+    import torch
+    inc = os.path.join(os.path.dirname(torch.__file__), "include")
+    tlib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    tmp = HOST_OUT + ".tmp"
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-DUSE_ROCM", "-D__HIP_PLATFORM_AMD__",
+           "-I" + os.path.join(ROOT, "include"), "-isystem", inc, "-isystem",
+           os.path.join(inc, "torch", "csrc", "api", "include"), "-isystem", sysconfig.get_paths()["include"],
+           "-isystem", "/opt/rocm/include", HOST_SRC, "-o", tmp, "-L" + tlib, "-ltorch_python", "-ltorch_cpu",
+           "-ltorch", "-lc10", "-lc10_hip", "-L" + HERE, "-lbf16x_hip", "-Wl,-rpath,$ORIGIN"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("g++ failed on host_ext.cpp:\n" + r.stdout + r.stderr)
+    os.replace(tmp, HOST_OUT)
+
+
 def build(verbose: bool = False) -> str:
     os.makedirs(BUILD_DIR, exist_ok=True)
     srcs = sorted(glob.glob(os.path.join(CSRC, "*.hip")) + glob.glob(os.path.join(CSRC, "*.cpp")))
+    srcs.remove(HOST_SRC)
     with cf.ThreadPoolExecutor(max_workers=min(8, len(srcs))) as ex:
         objs = list(ex.map(lambda s: _compile(s, verbose), srcs))
     tmp = OUT + ".tmp"
@@ -69,6 +95,7 @@ def build(verbose: bool = False) -> str:
     if r.returncode != 0:
         raise RuntimeError("link failed:\n" + r.stdout + r.stderr)
     os.replace(tmp, OUT)
+    _build_host(verbose)
     return OUT
 
 

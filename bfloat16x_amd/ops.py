@@ -11,6 +11,7 @@ a missing library or a CPU tensor raises.
 from __future__ import annotations
 
 import collections
+import functools
 
 import torch
 
@@ -134,10 +135,9 @@ def bf16x_decode(sign, mant, delta, emax, out_f, in_f, ovf_idx=None, ovf_val=Non
         out = torch.empty(out_f, in_f, dtype=torch.bfloat16, device=s.device)
     else:
         _out(out, out_f * in_f, s.device)
-    st = _lib.lib().bf16x_decode(s.data_ptr(), s.numel(), m.data_ptr(), m.numel(), d.data_ptr(), d.numel(),
-                                 e.data_ptr(), e.numel(), _lib.ptr(plan.tile_off) if plan else None,
-                                 _lib.ptr(plan.tile_ent) if plan else None, out_f, in_f, int(sub), mode,
-                                 out.data_ptr(), _lib.stream_of(s.device))
+    st = _lib.host().bf16x_decode(s, s.numel(), m, m.numel(), d, d.numel(), e, e.numel(),
+                                  plan.tile_off if plan else None, plan.tile_ent if plan else None, out_f, in_f,
+                                  int(sub), mode, out, _lib.stream_of(s.device))
     _lib.check(st, "bf16x_decode")
     return out
 
@@ -149,6 +149,15 @@ def bf16x_gemv(x, sign, mant, delta, emax, out_f, in_f, plan: Bf16xPlan | None =
                out: torch.Tensor | None = None) -> torch.Tensor:
     """y[out_f] (bf16) = W . x with W decoded on the fly; exact with a plan,
     saturated without one."""
+    # ordinary tensors: checks, output and launch in one native call
+    y = None
+    if plan is None:
+        y = _lib.host().gemv(x, sign, mant, delta, emax, None, None, None, out_f, in_f, sub, out)
+    elif plan.out_f == out_f and plan.in_f == in_f:
+        y = _lib.host().gemv(x, sign, mant, delta, emax, plan.tile_off, plan.tile_ent, plan.tile_sat, out_f, in_f,
+                             sub, out)
+    if y is not None:
+        return y
     s, m, d, e = _streams(sign, mant, delta, emax)
     xx = _dev_tensor(x, "x", tuple(_X_DTYPES)).reshape(-1)
     out_f, in_f = int(out_f), int(in_f)
@@ -331,7 +340,9 @@ GEMM_CHUNKS_MAX_IN_F = 8192
 GEMM_CHUNKS_LARGE = 1 << 26
 
 
+@functools.lru_cache(maxsize=None)
 def _cus(dev) -> int:
+    """Compute units of a device (a constant of the machine)."""
     return torch.cuda.get_device_properties(dev).multi_processor_count
 
 
@@ -350,31 +361,26 @@ GEMM_ONE_ROW_GEMV = True
 
 def _gemm_launch(x2, s, m, d, e, out_f, in_f, plan, y, y_dtype, sub=16):
     mode = _lib.SATURATED if plan is None else _lib.EXACT
-    L = _lib.lib()
+    H = _lib.host()
     M = x2.shape[0]
     if M <= GEMM_ROWS_MAX and in_f in GEMM_ROWS_IN_F:
-        st = L.bf16x_gemm_rows(x2.data_ptr(), _lib.BF16, M, s.data_ptr(), s.numel(), m.data_ptr(),
-                               m.numel(), d.data_ptr(), d.numel(), e.data_ptr(), e.numel(),
-                               _lib.ptr(plan.tile_off) if plan is not None else None,
-                               _lib.ptr(plan.tile_ent) if plan is not None else None, out_f, in_f, int(sub),
-                               mode, y.data_ptr(), y_dtype, _lib.stream_of(s.device))
+        st = H.bf16x_gemm_rows(x2, _lib.BF16, M, s, s.numel(), m, m.numel(), d, d.numel(), e, e.numel(),
+                               plan.tile_off if plan is not None else None,
+                               plan.tile_ent if plan is not None else None, out_f, in_f, int(sub), mode, y, y_dtype,
+                               _lib.stream_of(s.device))
         _lib.check(st, "bf16x_gemm_rows")
         return
     if _use_chunks(M, out_f, in_f, x2.device):
         cp_off, cp_ent = plan.cplan() if plan is not None else (None, None)
-        st = L.bf16x_gemm_chunks(x2.data_ptr(), _lib.BF16, M, s.data_ptr(), s.numel(), m.data_ptr(),
-                                 m.numel(), d.data_ptr(), d.numel(), e.data_ptr(), e.numel(), _lib.ptr(cp_off),
-                                 _lib.ptr(cp_ent), out_f, in_f, int(sub), mode, y.data_ptr(), y_dtype,
-                                 _lib.stream_of(s.device))
+        st = H.bf16x_gemm_chunks(x2, _lib.BF16, M, s, s.numel(), m, m.numel(), d, d.numel(), e, e.numel(), cp_off,
+                                 cp_ent, out_f, in_f, int(sub), mode, y, y_dtype, _lib.stream_of(s.device))
         _lib.check(st, "bf16x_gemm_chunks")
         return
     kp_off, kp_ent = plan.kplan() if plan is not None else (None, None)
-    ws_bytes = int(L.bf16x_gemm_workspace(M, out_f, in_f))
+    ws_bytes = int(_lib.lib().bf16x_gemm_workspace(M, out_f, in_f))
     ws = torch.empty((ws_bytes + 3) // 4, dtype=torch.float32, device=x2.device) if ws_bytes else None
-    st = L.bf16x_gemm(x2.data_ptr(), _lib.BF16, M, s.data_ptr(), s.numel(), m.data_ptr(),
-                      m.numel(), d.data_ptr(), d.numel(), e.data_ptr(), e.numel(), _lib.ptr(kp_off),
-                      _lib.ptr(kp_ent), out_f, in_f, int(sub), mode, y.data_ptr(), y_dtype,
-                      _lib.ptr(ws), ws_bytes, _lib.stream_of(s.device))
+    st = H.bf16x_gemm(x2, _lib.BF16, M, s, s.numel(), m, m.numel(), d, d.numel(), e, e.numel(), kp_off, kp_ent,
+                      out_f, in_f, int(sub), mode, y, y_dtype, ws, ws_bytes, _lib.stream_of(s.device))
     _lib.check(st, "bf16x_gemm")
 
 
@@ -383,20 +389,21 @@ def _gemm_terms(x2, s, m, d, e, out_f, in_f, plan, sub):
     (exact for fp16, 16 significant bits for fp32), the products in fp32.
     The terms are the 2 M rows of one launch, which decodes W once for both;
     where 2 M rows pass the kernels' 32-bit offsets, one launch each."""
-    L = _lib.lib()
-    M, dev, st = x2.shape[0], x2.device, _lib.stream_of(x2.device)
-    terms = torch.empty(2, M, in_f, dtype=torch.bfloat16, device=dev)
-    _lib.check(L.bf16x_split_terms(x2.data_ptr(), _X_DTYPES[x2.dtype], x2.numel(), terms[0].data_ptr(),
-                                   terms[1].data_ptr(), st), "bf16x_split_terms")
-    parts = torch.empty(2, M, out_f, dtype=torch.float32, device=dev)
+    H = _lib.host()
+    M, dev, st, code = x2.shape[0], x2.device, _lib.stream_of(x2.device), _X_DTYPES[x2.dtype]
+    terms = torch.empty(2 * M, in_f, dtype=torch.bfloat16, device=dev)
+    hi = terms.data_ptr()
+    _lib.check(H.bf16x_split_terms(x2, code, M * in_f, hi, hi + 2 * M * in_f, st), "bf16x_split_terms")
+    parts = torch.empty(2 * M, out_f, dtype=torch.float32, device=dev)
     if 2 * M * in_f * 2 < 0xFFFFFFFF:
-        _gemm_launch(terms.view(2 * M, in_f), s, m, d, e, out_f, in_f, plan, parts.view(2 * M, out_f), _lib.F32, sub)
+        _gemm_launch(terms, s, m, d, e, out_f, in_f, plan, parts, _lib.F32, sub)
     else:
         for k in range(2):
-            _gemm_launch(terms[k], s, m, d, e, out_f, in_f, plan, parts[k], _lib.F32, sub)
+            _gemm_launch(terms[k * M:(k + 1) * M], s, m, d, e, out_f, in_f, plan, parts[k * M:(k + 1) * M], _lib.F32,
+                         sub)
     y = torch.empty(M, out_f, dtype=x2.dtype, device=dev)
-    _lib.check(L.bf16x_add_terms(parts[0].data_ptr(), parts[1].data_ptr(), y.numel(), y.data_ptr(),
-                                 _X_DTYPES[y.dtype], st), "bf16x_add_terms")
+    a = parts.data_ptr()
+    _lib.check(H.bf16x_add_terms(a, a + 4 * M * out_f, M * out_f, y, code, st), "bf16x_add_terms")
     return y
 
 
@@ -443,9 +450,12 @@ def bf16x_gemm(x, sign, mant, delta, emax, out_f, in_f, plan: Bf16xPlan | None =
     not take (in_f not a multiple of 64, or above 65536), "fused" otherwise."""
     if path not in ("auto", "fused", "decode"):
         raise ValueError(f"path must be auto, fused or decode, not {path!r}")
-    s, m, d, e = _streams(sign, mant, delta, emax)
     out_f, in_f = int(out_f), int(in_f)
-    xx = _on(_dev_tensor(x, "x", tuple(_X_DTYPES)), s.device, "x")
+    if _lib.host().plain(x, sign, mant, delta, emax):      # nothing to convert or refuse
+        s, m, d, e, xx = sign, mant, delta, emax, x
+    else:
+        s, m, d, e = _streams(sign, mant, delta, emax)
+        xx = _on(_dev_tensor(x, "x", tuple(_X_DTYPES)), s.device, "x")
     if xx.shape[-1] != in_f:
         raise ValueError(f"x has last dimension {xx.shape[-1]}, in_f = {in_f}")
     _plan_on(plan, s.device, out_f, in_f)
