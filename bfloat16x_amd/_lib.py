@@ -61,6 +61,9 @@ PROTOTYPES = {
     "bf16x_cplan_build": (ctypes.c_int, [_P, _P, _c_i64, _c_i64, _P, _P, _P]),
     "bf16x_gemm_chunks": (ctypes.c_int, [_P, _c_i32, _c_i64, _P, _c_i64, _P, _c_i64, _P, _c_i64, _P, _c_i64, _P,
                                          _P, _c_i64, _c_i64, _c_i32, _c_i32, _P, _c_i32, _P]),
+    "bf16x_gemm_terms_workspace": (_c_i64, [_c_i64, _c_i64, _c_i64]),
+    "bf16x_gemm_terms": (ctypes.c_int, [_P, _c_i32, _c_i64, _P, _c_i64, _P, _c_i64, _P, _c_i64, _P, _c_i64, _P, _P,
+                                        _c_i64, _c_i64, _c_i32, _c_i32, _P, _P, _c_i64, _P]),
     "bf16x_split_terms": (ctypes.c_int, [_P, _c_i32, _c_i64, _P, _P, _P]),
     "bf16x_add_terms": (ctypes.c_int, [_P, _P, _c_i64, _P, _c_i32, _P]),
     "bf16x_fp32_to_bf16_host": (ctypes.c_int, [_P, _c_i64, _P, _c_i32]),

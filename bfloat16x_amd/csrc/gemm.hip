@@ -483,8 +483,8 @@ extern "C" int bf16x_gguf_kplan_build(const uint32_t* row_off, const uint32_t* e
 }
 
 // wave-specialised kernel (gemm_ws.hip): M >= ws_rows()
-int64_t bf16x_gemm_ws_workspace(int64_t M, int64_t out_f, int64_t in_f);
-int bf16x_gemm_ws_launch(const uint16_t* x, int64_t M, const uint32_t* s, const uint32_t* m, const uint32_t* d,
+int64_t bf16x_gemm_ws_workspace(int64_t M, int64_t out_f, int64_t in_f, bool terms);
+int bf16x_gemm_ws_launch(const void* x, int32_t x_dtype, int64_t M, const uint32_t* s, const uint32_t* m, const uint32_t* d,
                          const uint16_t* e, const uint8_t* blocks, const uint32_t* kp_off, const uint32_t* kp_ent,
                          int64_t out_f, int64_t in_f, bool exact, bool yf32, void* y, void* workspace,
                          int64_t workspace_bytes, hipStream_t st);
@@ -587,7 +587,7 @@ extern "C" int64_t bf16x_gemm_workspace(int64_t M, int64_t out_f, int64_t in_f) 
   if (M <= 0 || out_f <= 0 || in_f < kBK) return 0;
   if (use_skinny2(M, out_f, in_f)) return bf16x_gemm_skinny2_workspace(M, out_f, in_f);
   if (M <= skinny_rows()) return 0;
-  if (use_ws(M, out_f, in_f)) return bf16x_gemm_ws_workspace(M, out_f, in_f);
+  if (use_ws(M, out_f, in_f)) return bf16x_gemm_ws_workspace(M, out_f, in_f, false);
   const GemmShape g = gemm_shape(M, out_f, in_f);
   return g.nsplit > 1 ? (int64_t)g.nsplit * M * out_f * 4 : 0;
 }
@@ -623,7 +623,7 @@ extern "C" int bf16x_gemm(const void* x, int32_t x_dtype, int64_t M, const int32
     return rc ? rc : launch_status();
   }
   if (use_ws(M, out_f, in_f)) {
-    rc = bf16x_gemm_ws_launch((const uint16_t*)x, M, (const uint32_t*)sign, (const uint32_t*)mant,
+    rc = bf16x_gemm_ws_launch(x, BF16X_BF16, M, (const uint32_t*)sign, (const uint32_t*)mant,
                               (const uint32_t*)delta, (const uint16_t*)emax, nullptr, kp_off, kp_ent, out_f, in_f,
                               mode == BF16X_EXACT, y_dtype == BF16X_F32, y, workspace, workspace_bytes, st);
     return rc ? rc : launch_status();
@@ -677,4 +677,36 @@ extern "C" int bf16x_gemm(const void* x, int32_t x_dtype, int64_t M, const int32
                          count, g.nsplit, y);
   }
   return launch_status();
+}
+
+// fp16 / fp32 activations as two bf16 terms, where the 2 M rows of the terms
+// would run on the grouped wave-specialised kernel (which then takes both
+// terms into one accumulator); BF16X_ESHAPE elsewhere.
+extern "C" int64_t bf16x_gemm_terms_workspace(int64_t M, int64_t out_f, int64_t in_f) {
+  if (M <= 0 || out_f <= 0 || in_f < kBK || (in_f % kBK) != 0) return BF16X_ESHAPE;
+  if (!ws_groups(in_f) || !use_ws(2 * M, out_f, in_f) || tiles_per_row(in_f) != 1) return BF16X_ESHAPE;
+  // 32-bit buffer offsets, as in bf16x_gemm
+  if (out_f * (in_f >> 5) * 28 >= (int64_t)0xFFFFFFFF || 2 * M * in_f * 2 >= (int64_t)0xFFFFFFFF) return BF16X_ESHAPE;
+  return bf16x_gemm_ws_workspace(M, out_f, in_f, true);
+}
+
+extern "C" int bf16x_gemm_terms(const void* x, int32_t x_dtype, int64_t M, const int32_t* sign, int64_t n_sign,
+                                const int32_t* mant, int64_t n_mant, const int32_t* delta, int64_t n_delta,
+                                const uint8_t* emax, int64_t n_emax, const uint32_t* kp_off, const uint32_t* kp_ent,
+                                int64_t out_f, int64_t in_f, int32_t sub, int32_t mode, void* y, void* workspace,
+                                int64_t workspace_bytes, bf16x_stream_t stream) {
+  if (!x || !sign || !mant || !delta || !emax || !y) return BF16X_EARG;
+  if (mode != BF16X_EXACT && mode != BF16X_SATURATED) return BF16X_EARG;
+  if (mode == BF16X_EXACT && (!kp_off || !kp_ent)) return BF16X_EARG;
+  if (x_dtype != BF16X_F16 && x_dtype != BF16X_F32) return BF16X_EDTYPE;
+  if (M <= 0) return BF16X_ESHAPE;
+  const int rc = check_dict(out_f, in_f, sub, n_sign, n_mant, n_delta, n_emax);
+  if (rc) return rc;
+  if (bf16x_gemm_terms_workspace(M, out_f, in_f) < 0) return BF16X_ESHAPE;
+  if (!aligned4(sign) || !aligned4(mant) || !aligned4(delta) || !aligned2(emax) || !aligned4(x) ||
+      !(x_dtype == BF16X_F16 ? aligned2(y) : aligned4(y)))
+    return BF16X_EARG;
+  return bf16x_gemm_ws_launch(x, x_dtype, M, (const uint32_t*)sign, (const uint32_t*)mant, (const uint32_t*)delta,
+                              (const uint16_t*)emax, nullptr, kp_off, kp_ent, out_f, in_f, mode == BF16X_EXACT,
+                              x_dtype == BF16X_F32, y, workspace, workspace_bytes, (hipStream_t)stream);
 }

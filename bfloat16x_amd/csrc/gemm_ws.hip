@@ -146,7 +146,15 @@ __device__ __forceinline__ WsWork ws_work(const WsGrid& g, int units) {
 // columns past out_f hold zeros), in K-range order.  The wave owns NT 32-token
 // tiles from token 32 NT (wave % TG) and NJ 32-row W tiles from row
 // 32 NJ (wave / TG).
-template <bool YF32, int NT, int TG, int NJ>
+enum { kYBf16 = 0, kYF32 = 1, kYF16 = 2 };     // output types of the kernels below
+template <int YT>
+__device__ __forceinline__ void store_y(void* __restrict__ y, int64_t i, float v) {
+  if constexpr (YT == kYF32) ((float*)y)[i] = v;
+  else if constexpr (YT == kYF16) ((_Float16*)y)[i] = (_Float16)v;
+  else ((uint16_t*)y)[i] = (uint16_t)f32_to_bf16_rne(v);
+}
+
+template <int YT, int NT, int TG, int NJ>
 __device__ __forceinline__ void ws_store(const f32x16 (&acc)[NT][NJ], const WsWork& w, int wave, int lane, int64_t M,
                                          int64_t out_f, int ltiles, void* __restrict__ y, float* __restrict__ part) {
   constexpr int BM = 32 * NT * TG;
@@ -173,10 +181,7 @@ __device__ __forceinline__ void ws_store(const f32x16 (&acc)[NT][NJ], const WsWo
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
         const int64_t row = w.m0 + t0 + i * 32 + 8 * (v >> 2) + 4 * h + (v & 3);
-        if (row < M && col < out_f) {
-          if constexpr (YF32) ((float*)y)[row * out_f + col] = acc[i][jj][v];
-          else ((uint16_t*)y)[row * out_f + col] = (uint16_t)f32_to_bf16_rne(acc[i][jj][v]);
-        }
+        if (row < M && col < out_f) store_y<YT>(y, row * out_f + col, acc[i][jj][v]);
       }
     }
   }
@@ -446,7 +451,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     step(j + 1, 1, X1, X0);
   }
   if (j < n) step(j, 0, X0, X1);
-  ws_store<YF32, 2, 4, 4>(acc, wk, wave, lane, M, out_f, grid.ltiles, y, part);
+  ws_store<YF32 ? kYF32 : kYBf16, 2, 4, 4>(acc, wk, wave, lane, M, out_f, grid.ltiles, y, part);
 }
 
 // ---------------------------------------------------------------------------
@@ -486,7 +491,7 @@ constexpr int kWSlot4 = kBN * kRowB4;        // 64 KB
 
 __device__ __forceinline__ int swz4(int row, int chunk) { return chunk ^ (((chunk >> 4) & 1) << 1) ^ (row & 15); }
 
-template <bool GG, bool EXACT, bool YF32, int NT, int TG, int ND>
+template <bool GG, bool EXACT, int YT, int NT, int TG, int ND, int NX>
 __global__ __launch_bounds__(64 * (4 + ND)) __attribute__((amdgpu_waves_per_eu((4 + ND) / 4, (4 + ND) / 4)))
 void gemm_ws4_kernel(
     const uint16_t* __restrict__ x, int64_t M, const uint32_t* __restrict__ sign,
@@ -726,36 +731,46 @@ void gemm_ws4_kernel(
   constexpr int NM = NT * NJ;                 // MFMAs per k-quarter
   if constexpr (NT == 1) {
     // Few MFMAs per k-quarter: a quarter's operands are requested into the
-    // registers of the quarter just multiplied, WD steps (W, from LDS) and XD
-    // steps (x) ahead, so an LDS read has at least three quarters' MFMAs to
-    // arrive.  The group's last WD steps request the next group's operands:
-    // the barrier comes before them, when all of this group's are in
-    // registers, which also frees the slot for the decode waves early.
-    constexpr int WD = NJ == 4 ? 1 : 2, XD = WD;
-    bf16x8_t X[XD][4], W[WD][4][NJ];
-    auto load_xq = [&](int jx, int q, bf16x8_t& d) {
+    // registers of the quarter just multiplied, WQ quarters (W, from LDS) and
+    // XD steps (x) ahead, so an LDS read has at least eight MFMAs to arrive.
+    // The group's last WQ quarters request the next group's operands: the
+    // barrier comes before them, when all of this group's are in registers,
+    // which also frees the slot for the decode waves early.
+    // NX = 2: x is two terms (hi, lo), both multiplied into the accumulator
+    // (4096x4096 fp16 M = 64: 21.5 us for the call, 30.1 with the terms split
+    // into 2 M rows and their results added by launches of their own).
+    constexpr int WQ = NX == 2 ? (NJ == 4 ? 2 : 4) : (NJ == 4 ? 4 : 8), XD = NJ == 4 || NX == 2 ? 1 : 2;
+    constexpr int kQ = 4 * kGroup;             // k-quarters of a group
+    bf16x8_t X[XD][4][NX], W[WQ][NJ];
+    const int64_t xrows = ((M + 31) / 32) * 32;
+    const __amdgpu_buffer_rsrc_t rlo_ =
+        rsrc(x + ((NX - 1) * xrows + m0) * in_f, (uint64_t)(xrows - m0) * (uint64_t)in_f * 2);
+    auto load_xq = [&](int jx, int q, bf16x8_t (&d)[NX]) {
       const uint32_t ks = (uint32_t)(s0 + min(jx, n - 1)) * 4096;
-      const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rx_, (int)(vx[0] + q * 1024), (int)ks, 0);
-      d = __builtin_bit_cast(bf16x8_t, v);
+#pragma unroll
+      for (int t = 0; t < NX; ++t) {
+        const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(t ? rlo_ : rx_, (int)(vx[0] + q * 1024), (int)ks, 0);
+        d[t] = __builtin_bit_cast(bf16x8_t, v);
+      }
     };
     auto group = [&](int jg, int slot) {
 #pragma unroll
-      for (int u = 0; u < kGroup; ++u) {
-        if (u == kGroup - WD) {
+      for (int p = 0; p < kQ; ++p) {
+        if (p == kQ - WQ) {
           __builtin_amdgcn_sched_barrier(0);
           __syncthreads();
           __builtin_amdgcn_sched_barrier(0);
         }
-        const int nu = (u + WD) % kGroup, ns = u + WD >= kGroup ? slot ^ 1 : slot;
+        const int u = p >> 2, q = p & 3, np = (p + WQ) % kQ;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
+        for (int t = 0; t < NX; ++t)
 #pragma unroll
           for (int jj = 0; jj < NJ; ++jj)
-            acc[0][jj] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(X[u % XD][q], W[u % WD][q][jj], acc[0][jj], 0, 0, 0);
-          load_xq(4 * jg + u + XD, q, X[u % XD][q]);
-          load_w(q, nu, ns, W[u % WD][q]);
-          __builtin_amdgcn_sched_barrier(0);
-        }
+            acc[0][jj] =
+                __builtin_amdgcn_mfma_f32_32x32x16_bf16(X[u % XD][q][t], W[p % WQ][jj], acc[0][jj], 0, 0, 0);
+        load_xq(4 * jg + u + XD, q, X[u % XD][q]);
+        load_w(np & 3, np >> 2, p + WQ >= kQ ? slot ^ 1 : slot, W[p % WQ]);
+        __builtin_amdgcn_sched_barrier(0);
       }
     };
 #pragma unroll
@@ -764,9 +779,7 @@ void gemm_ws4_kernel(
       for (int q = 0; q < 4; ++q) load_xq(u, q, X[u][q]);
     __syncthreads();
 #pragma unroll
-    for (int u = 0; u < WD; ++u)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) load_w(q, u, 0, W[u][q]);
+    for (int p = 0; p < WQ; ++p) load_w(p & 3, p >> 2, 0, W[p]);
     __builtin_amdgcn_sched_barrier(0);
     int jg = 0;
     for (; jg + 1 < ng; jg += 2) {
@@ -839,7 +852,7 @@ void gemm_ws4_kernel(
   }
   if (jg < ng) group(jg, 0);
   }
-  ws_store<YF32, NT, TG, NJ>(acc, wk, wave, lane, M, out_f, grid.ltiles, y, part);
+  ws_store<YT, NT, TG, NJ>(acc, wk, wave, lane, M, out_f, grid.ltiles, y, part);
 }
 
 // x [M, K] -> operand order: 32-row tile T, step s (64 columns), k-quarter q
@@ -847,40 +860,79 @@ void gemm_ws4_kernel(
 // 32 T + lr, columns 64 s + 32 h + {4q, 16+4q, 4q+1, 17+4q, .., 4q+3, 19+4q}
 // (the MFMA A operand of the fused kernels, in the K order of the W tile).
 // Rows past M (up to the 32-row boundary) are zeros.  One thread per
-// (T, s, l): it reads the 64 contiguous bytes of its row's 32 columns (lanes
-// l and l + 32 take the two halves of a 128-byte row segment) and writes its
-// 16 bytes of each of the 4 k-quarters (each a contiguous 1 KB per wave).
-__global__ __launch_bounds__(256) void x_op_kernel(const uint16_t* __restrict__ x, int64_t M, int64_t in_f,
+// (T, s, l): it reads the 32 contiguous columns of its row (lanes l and l + 32
+// take the two halves of a 64-column row segment) and writes its 16 bytes of
+// each of the 4 k-quarters (each a contiguous 1 KB per wave).  XT fp16 or
+// fp32: two such matrices, hi = bf16(x) and, behind it, lo = bf16(x - hi).
+__device__ __forceinline__ void xo_store(const uint32_t (&w)[16], u32x4* __restrict__ xo, int64_t ts, int l) {
+  // quarter q: columns 4q .. 4q+3 (words 2q, 2q+1) and 16+4q .. 19+4q (words 8+2q, 9+2q)
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    xo[(ts * 4 + q) * 64 + l] = u32x4{perm(w[8 + 2 * q], w[2 * q], 0x05040100u),
+                                      perm(w[8 + 2 * q], w[2 * q], 0x07060302u),
+                                      perm(w[9 + 2 * q], w[2 * q + 1], 0x05040100u),
+                                      perm(w[9 + 2 * q], w[2 * q + 1], 0x07060302u)};
+}
+template <int XT>
+__global__ __launch_bounds__(256) void x_op_kernel(const void* __restrict__ x, int64_t M, int64_t in_f,
                                                    int64_t units, u32x4* __restrict__ xo) {
   const int64_t S = in_f / 64;
   for (int64_t u = (int64_t)blockIdx.x * 256 + threadIdx.x; u < units; u += (int64_t)gridDim.x * 256) {
     const int l = (int)(u & 63);
     const int64_t ts = u >> 6, T = ts / S, s = ts - T * S;
     const int64_t row = T * 32 + (l & 31);
+    const int64_t e0 = row * in_f + s * 64 + (l >> 5) * 32;
     uint32_t w[16] = {0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u};
-    if (row < M) {
-      const u32x4a* src = (const u32x4a*)(x + row * in_f + s * 64 + (l >> 5) * 32);
+    if constexpr (XT == BF16X_BF16) {
+      if (row < M) {
+        const u32x4a* src = (const u32x4a*)((const uint16_t*)x + e0);
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const u32x4a v = src[c];
-        const uint32_t v0 = v.x, v1 = v.y, v2 = v.z, v3 = v.w;
-        w[4 * c] = v0; w[4 * c + 1] = v1; w[4 * c + 2] = v2; w[4 * c + 3] = v3;
+        for (int c = 0; c < 4; ++c) {
+          const u32x4a v = src[c];
+          const uint32_t v0 = v.x, v1 = v.y, v2 = v.z, v3 = v.w;
+          w[4 * c] = v0; w[4 * c + 1] = v1; w[4 * c + 2] = v2; w[4 * c + 3] = v3;
+        }
       }
-    }
-    // quarter q: columns 4q .. 4q+3 (words 2q, 2q+1) and 16+4q .. 19+4q (words 8+2q, 9+2q)
+      xo_store(w, xo, ts, l);
+    } else {
+      uint32_t lo[16] = {0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u};
+      if (row < M) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
-      xo[(ts * 4 + q) * 64 + l] = u32x4{perm(w[8 + 2 * q], w[2 * q], 0x05040100u),
-                                        perm(w[8 + 2 * q], w[2 * q], 0x07060302u),
-                                        perm(w[9 + 2 * q], w[2 * q + 1], 0x05040100u),
-                                        perm(w[9 + 2 * q], w[2 * q + 1], 0x07060302u)};
+        for (int k = 0; k < 16; ++k) {
+          float f[2];
+          if constexpr (XT == BF16X_F16) {
+            const uint32_t v = ((const u32x4a*)((const _Float16*)x + e0))[k >> 2][k & 3];
+            typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+            f16x2 h;
+            __builtin_memcpy(&h, &v, 4);
+            f[0] = (float)h.x;
+            f[1] = (float)h.y;
+          } else {
+            const u32x4a v = ((const u32x4a*)((const float*)x + e0))[k >> 1];
+            const uint32_t a = k & 1 ? v.z : v.x, b = k & 1 ? v.w : v.y;
+            f[0] = __uint_as_float(a);
+            f[1] = __uint_as_float(b);
+          }
+          uint32_t h[2], r[2];
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            h[i] = f32_to_bf16_rne(f[i]);
+            r[i] = f32_to_bf16_rne(f[i] - __uint_as_float(h[i] << 16));
+          }
+          w[k] = h[0] | (h[1] << 16);
+          lo[k] = r[0] | (r[1] << 16);
+        }
+      }
+      xo_store(w, xo, ts, l);
+      xo_store(lo, xo + units * 4, ts, l);
+    }
   }
 }
 
 // y over the split tiles: the sum of each element's fp32 partials in K-range
 // order (partial tile layout as ws_store writes it).  One thread per element
 // of the split tiles' 256 x 128 partials, in order.
-template <bool YF32>
+template <int YT>
 __global__ __launch_bounds__(256) void ws_tile_reduce_kernel(const float* __restrict__ part, WsGrid g, int nsplit,
                                                              int64_t M, int64_t out_f, void* __restrict__ y,
                                                              bool yal) {
@@ -901,18 +953,18 @@ __global__ __launch_bounds__(256) void ws_tile_reduce_kernel(const float* __rest
     const float v[4] = {s.x, s.y, s.z, s.w};
     const int64_t o = row * out_f + col;
     if (yal && col + 3 < out_f && (o & 3) == 0) {
-      if constexpr (YF32) {
+      if constexpr (YT == kYF32) {
         *(f32x4v*)((float*)y + o) = s;
+      } else if constexpr (YT == kYF16) {
+        typedef _Float16 f16x4v __attribute__((ext_vector_type(4)));
+        *(f16x4v*)((_Float16*)y + o) = f16x4v{(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
       } else {
         const uint32_t lo = f32_to_bf16_rne(v[0]) | (f32_to_bf16_rne(v[1]) << 16);
         const uint32_t hi = f32_to_bf16_rne(v[2]) | (f32_to_bf16_rne(v[3]) << 16);
         *(u32x2a*)((uint16_t*)y + o) = u32x2a{lo, hi};
       }
     } else {
-      for (int c = 0; c < 4 && col + c < out_f; ++c) {
-        if constexpr (YF32) ((float*)y)[o + c] = v[c];
-        else ((uint16_t*)y)[o + c] = (uint16_t)f32_to_bf16_rne(v[c]);
-      }
+      for (int c = 0; c < 4 && col + c < out_f; ++c) store_y<YT>(y, o + c, v[c]);
     }
   }
 }
@@ -951,14 +1003,14 @@ int64_t ws_resident() {
 // 42.1 / 48.7, M = 128 52.8 / 45.3 / 51.1, M = 191 74.9 / 60.7 / 54.3;
 // 4096x4096 (32 row tiles) M = 64 22.6 / 24.1 / 28.8, M = 128 23.8 / 24.9 /
 // 29.5, M = 191 30.1 / 27.3 / 30.7.
-int64_t ws_tile_rows(int64_t M, int64_t nt, int64_t C) {
+int64_t ws_tile_rows(int64_t M, int64_t nt, int64_t C, bool terms) {
   const int64_t t = tuning(BF16X_TUNE_GEMM_WS_BM);
-  if (t == 64 || t == 128 || t == 256) return t;
+  if (t == 64 || t == 128 || (t == 256 && !terms)) return t;
   for (int64_t bm = 64; bm < 256; bm *= 2) {
     const int64_t mt = (M + bm - 1) / bm;
     if (mt == 1 || (mt == 2 && mt * nt <= C / 4)) return bm;
   }
-  return 256;
+  return terms ? 128 : 256;    // two terms: the operands of a 256-token tile do not fit the registers
 }
 
 // Tiles run whole-K in full rounds of resident blocks; the f tiles of the
@@ -970,13 +1022,13 @@ int64_t ws_tile_rows(int64_t M, int64_t nt, int64_t C) {
 // only for those 128 tiles.  BF16X_TUNE_GEMM_WS_SPLIT > 0 splits every tile
 // into that many K ranges instead; BF16X_TUNE_GEMM_WS_RESIDENT > 0 replaces
 // the resident block count (tests reach the mixed plan with few tiles).
-WsShape ws_shape(int64_t M, int64_t out_f, int64_t in_f) {
+WsShape ws_shape(int64_t M, int64_t out_f, int64_t in_f, bool terms = false) {
   WsShape w;
   w.grouped = ws_grouped(in_f);
   const int64_t forced_c = tuning(BF16X_TUNE_GEMM_WS_RESIDENT);
   const int64_t C = forced_c > 0 ? forced_c : ws_resident();
   const int64_t nt = (out_f + kBN - 1) / kBN;
-  const int64_t bm = w.grouped ? ws_tile_rows(M, nt, C) : kBM;
+  const int64_t bm = w.grouped ? ws_tile_rows(M, nt, C, terms) : kBM;
   const int64_t mt = (M + bm - 1) / bm;
   const int64_t S = in_f / kStep, tiles = mt * nt;
   const int64_t units = w.grouped ? S / kGroup : S;
@@ -1010,41 +1062,56 @@ namespace {
 int64_t ws_xop_bytes(int64_t M, int64_t in_f) { return ((M + 31) / 32) * 32 * in_f * 2; }
 }  // namespace
 
-int64_t bf16x_gemm_ws_workspace(int64_t M, int64_t out_f, int64_t in_f) {
-  const WsShape w = ws_shape(M, out_f, in_f);
-  return ws_xop_bytes(M, in_f) + (w.nsplit > 1 ? (int64_t)w.nsplit * w.g.ltiles * ((int64_t)w.g.bm * kBN) * 4 : 0);
+// terms: x is fp16 or fp32, multiplied as two bf16 terms (grouped kernel only)
+int64_t bf16x_gemm_ws_workspace(int64_t M, int64_t out_f, int64_t in_f, bool terms) {
+  const WsShape w = ws_shape(M, out_f, in_f, terms);
+  return ws_xop_bytes(M, in_f) * (terms ? 2 : 1) +
+         (w.nsplit > 1 ? (int64_t)w.nsplit * w.g.ltiles * ((int64_t)w.g.bm * kBN) * 4 : 0);
 }
 
 // Launch of the wave-specialised kernel; arguments checked by the caller
-// (bf16x_gemm for the packed dict; bf16x_gguf_gemm for GGUF blocks, given
-// as `blocks` with the dict pointers null).
-int bf16x_gemm_ws_launch(const uint16_t* x, int64_t M, const uint32_t* s, const uint32_t* m, const uint32_t* d,
-                         const uint16_t* e, const uint8_t* blocks, const uint32_t* kp_off, const uint32_t* kp_ent,
-                         int64_t out_f, int64_t in_f, bool exact, bool yf32, void* y, void* workspace,
-                         int64_t workspace_bytes, hipStream_t st) {
-  const WsShape w = ws_shape(M, out_f, in_f);
+// (bf16x_gemm and bf16x_gemm_terms for the packed dict; bf16x_gguf_gemm for
+// GGUF blocks, given as `blocks` with the dict pointers null).  x_dtype fp16
+// or fp32: two terms, y in x's type; otherwise yf32 says bf16 or fp32.
+int bf16x_gemm_ws_launch(const void* x, int32_t x_dtype, int64_t M, const uint32_t* s, const uint32_t* m,
+                         const uint32_t* d, const uint16_t* e, const uint8_t* blocks, const uint32_t* kp_off,
+                         const uint32_t* kp_ent, int64_t out_f, int64_t in_f, bool exact, bool yf32, void* y,
+                         void* workspace, int64_t workspace_bytes, hipStream_t st) {
+  const bool terms = x_dtype != BF16X_BF16;
+  const WsShape w = ws_shape(M, out_f, in_f, terms);
+  if (terms && (!w.grouped || blocks)) return BF16X_ESHAPE;
   const int64_t xop = ws_xop_bytes(M, in_f);
-  if (!workspace || !aligned16(workspace) || workspace_bytes < bf16x_gemm_ws_workspace(M, out_f, in_f))
+  if (!workspace || !aligned16(workspace) || workspace_bytes < bf16x_gemm_ws_workspace(M, out_f, in_f, terms))
     return BF16X_ECAPACITY;
   if (xop >= (int64_t)0xFFFFFFFF) return BF16X_ESHAPE;
   if (w.grid > INT32_MAX) return BF16X_ESHAPE;
   const int64_t units = xop / 64;   // (32-row tile, step, lane): 4 chunks of 16 bytes each
-  hipLaunchKernelGGL(x_op_kernel, dim3((unsigned)std::min<int64_t>((units + 255) / 256, 8192)), dim3(256), 0, st,
-                     x, M, in_f, units, (u32x4*)workspace);
+  const dim3 xg((unsigned)std::min<int64_t>((units + 255) / 256, 8192));
+  if (x_dtype == BF16X_F16)
+    hipLaunchKernelGGL(x_op_kernel<BF16X_F16>, xg, dim3(256), 0, st, x, M, in_f, units, (u32x4*)workspace);
+  else if (x_dtype == BF16X_F32)
+    hipLaunchKernelGGL(x_op_kernel<BF16X_F32>, xg, dim3(256), 0, st, x, M, in_f, units, (u32x4*)workspace);
+  else
+    hipLaunchKernelGGL(x_op_kernel<BF16X_BF16>, xg, dim3(256), 0, st, x, M, in_f, units, (u32x4*)workspace);
   const uint16_t* xo = (const uint16_t*)workspace;
-  float* part = (float*)((uint8_t*)workspace + xop);
+  float* part = (float*)((uint8_t*)workspace + xop * (terms ? 2 : 1));
   const dim3 grid((unsigned)w.grid);
-#define BF16X_WS4(GG_, EX_, YF_, NT_, TG_, ND_)                                                                   \
-  hipLaunchKernelGGL((gemm_ws4_kernel<GG_, EX_, YF_, NT_, TG_, ND_>), grid, dim3(64 * (4 + ND_)), 0, st, xo, M, s, m, \
-                     d, e, blocks, kp_off, kp_ent, out_f, in_f, w.g, y, part)
+#define BF16X_WS4(GG_, EX_, YT_, NT_, TG_, ND_, NX_)                                                               \
+  hipLaunchKernelGGL((gemm_ws4_kernel<GG_, EX_, YT_, NT_, TG_, ND_, NX_>), grid, dim3(64 * (4 + ND_)), 0, st, xo, M, \
+                     s, m, d, e, blocks, kp_off, kp_ent, out_f, in_f, w.g, y, part)
 #define BF16X_WS1(GG_, EX_, YF_)                                                                                   \
   do {                                                                                                           \
     if (!w.grouped)                                                                                              \
       hipLaunchKernelGGL((gemm_ws_kernel<GG_, EX_, YF_>), grid, dim3(512), 0, st, xo, M, s, m, d, e, blocks,        \
                          kp_off, kp_ent, out_f, in_f, w.g, y, part);                                              \
-    else if (w.g.bm == 64) BF16X_WS4(GG_, EX_, YF_, 1, 2, 8);                                                     \
-    else if (w.g.bm == 128) BF16X_WS4(GG_, EX_, YF_, 1, 4, 8);                                                    \
-    else BF16X_WS4(GG_, EX_, YF_, 2, 4, 4);                                                                       \
+    else if (w.g.bm == 64) BF16X_WS4(GG_, EX_, (YF_ ? kYF32 : kYBf16), 1, 2, 8, 1);                                \
+    else if (w.g.bm == 128) BF16X_WS4(GG_, EX_, (YF_ ? kYF32 : kYBf16), 1, 4, 8, 1);                               \
+    else BF16X_WS4(GG_, EX_, (YF_ ? kYF32 : kYBf16), 2, 4, 4, 1);                                                 \
+  } while (0)
+#define BF16X_WSX(EX_, YT_)                                 \
+  do {                                                      \
+    if (w.g.bm == 64) BF16X_WS4(false, EX_, YT_, 1, 2, 8, 2); \
+    else BF16X_WS4(false, EX_, YT_, 1, 4, 8, 2);            \
   } while (0)
 #define BF16X_WS(GG_)                                        \
   do {                                                       \
@@ -1056,20 +1123,29 @@ int bf16x_gemm_ws_launch(const uint16_t* x, int64_t M, const uint32_t* s, const 
       else BF16X_WS1(GG_, false, false);                     \
     }                                                        \
   } while (0)
-  if (blocks) BF16X_WS(true);
-  else BF16X_WS(false);
+  const int yt = terms ? (x_dtype == BF16X_F16 ? kYF16 : kYF32) : (yf32 ? kYF32 : kYBf16);
+  if (terms) {
+    if (yt == kYF16) { if (exact) BF16X_WSX(true, kYF16); else BF16X_WSX(false, kYF16); }
+    else { if (exact) BF16X_WSX(true, kYF32); else BF16X_WSX(false, kYF32); }
+  } else if (blocks) {
+    BF16X_WS(true);
+  } else {
+    BF16X_WS(false);
+  }
+#undef BF16X_WSX
 #undef BF16X_WS
 #undef BF16X_WS1
 #undef BF16X_WS4
   if (w.nsplit > 1) {
     const int64_t count = (int64_t)w.g.ltiles * ((int64_t)w.g.bm * kBN);
     const int64_t blocks_r = std::min<int64_t>((count / 4 + 255) / 256, 4096);
-    if (yf32)
-      hipLaunchKernelGGL(ws_tile_reduce_kernel<true>, dim3((unsigned)blocks_r), dim3(256), 0, st,
-                         (const float*)part, w.g, w.nsplit, M, out_f, y, aligned16(y));
-    else
-      hipLaunchKernelGGL(ws_tile_reduce_kernel<false>, dim3((unsigned)blocks_r), dim3(256), 0, st,
-                         (const float*)part, w.g, w.nsplit, M, out_f, y, aligned16(y));
+#define BF16X_RED(YT_)                                                                                            \
+  hipLaunchKernelGGL(ws_tile_reduce_kernel<YT_>, dim3((unsigned)blocks_r), dim3(256), 0, st, (const float*)part, w.g, \
+                     w.nsplit, M, out_f, y, aligned16(y))
+    if (yt == kYF32) BF16X_RED(kYF32);
+    else if (yt == kYF16) BF16X_RED(kYF16);
+    else BF16X_RED(kYBf16);
+#undef BF16X_RED
   }
   return launch_status();
 }

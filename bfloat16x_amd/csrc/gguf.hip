@@ -628,15 +628,15 @@ extern "C" int bf16x_gguf_gemv_lossless(const void* x, int32_t x_dtype, const ui
 // gemm_ws.hip with its block loader (46-byte blocks, zero-marker decode).
 // The lossless table enters as the step-major plan of bf16x_gguf_kplan_build.
 // ---------------------------------------------------------------------------
-int64_t bf16x_gemm_ws_workspace(int64_t M, int64_t out_f, int64_t in_f);
-int bf16x_gemm_ws_launch(const uint16_t* x, int64_t M, const uint32_t* s, const uint32_t* m, const uint32_t* d,
+int64_t bf16x_gemm_ws_workspace(int64_t M, int64_t out_f, int64_t in_f, bool terms);
+int bf16x_gemm_ws_launch(const void* x, int32_t x_dtype, int64_t M, const uint32_t* s, const uint32_t* m, const uint32_t* d,
                          const uint16_t* e, const uint8_t* blocks, const uint32_t* kp_off, const uint32_t* kp_ent,
                          int64_t out_f, int64_t in_f, bool exact, bool yf32, void* y, void* workspace,
                          int64_t workspace_bytes, hipStream_t st);
 
 extern "C" int64_t bf16x_gguf_gemm_workspace(int64_t M, int64_t out_f, int64_t in_f) {
   if (M <= 0 || out_f <= 0 || in_f < 64 || (in_f % 64) != 0) return 0;
-  return bf16x_gemm_ws_workspace(M, out_f, in_f);
+  return bf16x_gemm_ws_workspace(M, out_f, in_f, false);
 }
 
 extern "C" int bf16x_gguf_gemm(const void* x, int32_t x_dtype, int64_t M, const uint8_t* blocks, int64_t n_bytes,
@@ -653,7 +653,7 @@ extern "C" int bf16x_gguf_gemm(const void* x, int32_t x_dtype, int64_t M, const 
     return BF16X_ESHAPE;
   if (!aligned16(x) || !aligned4(blocks) || !aligned4(y)) return BF16X_EARG;
   if (kp_off && (!aligned4(kp_off) || !aligned4(kp_ent))) return BF16X_EARG;
-  rc = bf16x_gemm_ws_launch((const uint16_t*)x, M, nullptr, nullptr, nullptr, nullptr, blocks, kp_off, kp_ent, out_f,
+  rc = bf16x_gemm_ws_launch(x, BF16X_BF16, M, nullptr, nullptr, nullptr, nullptr, blocks, kp_off, kp_ent, out_f,
                             in_f, kp_off != nullptr, y_dtype == BF16X_F32, y, workspace, workspace_bytes,
                             (hipStream_t)stream);
   return rc ? rc : launch_status();

@@ -165,6 +165,7 @@ ENTRY(bf16x_decode)
 ENTRY(bf16x_gemm)
 ENTRY(bf16x_gemm_rows)
 ENTRY(bf16x_gemm_chunks)
+ENTRY(bf16x_gemm_terms)
 ENTRY(bf16x_split_terms)
 ENTRY(bf16x_add_terms)
 ENTRY(bf16x_gguf_gemv)
@@ -178,7 +179,7 @@ ENTRY(bf16x_gguf_decode_lossless)
 #define ENTRY(name) FAST(#name, c_##name)
 PyMethodDef methods[] = {FAST("gemv", gemv), FAST("plain", plain), FAST("stream", stream), ENTRY(bf16x_decode),
                          ENTRY(bf16x_gemm), ENTRY(bf16x_gemm_rows), ENTRY(bf16x_gemm_chunks),
-                         ENTRY(bf16x_split_terms), ENTRY(bf16x_add_terms), ENTRY(bf16x_gguf_gemv),
+                         ENTRY(bf16x_gemm_terms), ENTRY(bf16x_split_terms), ENTRY(bf16x_add_terms), ENTRY(bf16x_gguf_gemv),
                          ENTRY(bf16x_gguf_gemv_lossless), ENTRY(bf16x_gguf_gemm), ENTRY(bf16x_gguf_decode),
                          ENTRY(bf16x_gguf_decode_lossless), {nullptr, nullptr, 0, nullptr}};
 

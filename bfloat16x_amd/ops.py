@@ -387,10 +387,21 @@ def _gemm_launch(x2, s, m, d, e, out_f, in_f, plan, y, y_dtype, sub=16):
 def _gemm_terms(x2, s, m, d, e, out_f, in_f, plan, sub):
     """x2 (fp16 or fp32) . W^T in x2's dtype: x = hi + lo as two bf16 terms
     (exact for fp16, 16 significant bits for fp32), the products in fp32.
-    The terms are the 2 M rows of one launch, which decodes W once for both;
-    where 2 M rows pass the kernels' 32-bit offsets, one launch each."""
+    Where 2 M rows would run on the grouped wave-specialised kernel, that
+    kernel takes both terms itself (bf16x_gemm_terms); elsewhere the terms are
+    the 2 M rows of one launch, which decodes W once for both, or where 2 M
+    rows pass the kernels' 32-bit offsets one launch each."""
     H = _lib.host()
     M, dev, st, code = x2.shape[0], x2.device, _lib.stream_of(x2.device), _X_DTYPES[x2.dtype]
+    ws_bytes = int(_lib.lib().bf16x_gemm_terms_workspace(M, out_f, in_f))
+    if ws_bytes > 0 and x2.data_ptr() % 4 == 0:
+        kp_off, kp_ent = plan.kplan() if plan is not None else (None, None)
+        ws = torch.empty((ws_bytes + 3) // 4, dtype=torch.float32, device=dev)
+        y = torch.empty(M, out_f, dtype=x2.dtype, device=dev)
+        _lib.check(H.bf16x_gemm_terms(x2, code, M, s, s.numel(), m, m.numel(), d, d.numel(), e, e.numel(), kp_off,
+                                      kp_ent, out_f, in_f, int(sub), _lib.SATURATED if plan is None else _lib.EXACT,
+                                      y, ws, ws_bytes, st), "bf16x_gemm_terms")
+        return y
     terms = torch.empty(2 * M, in_f, dtype=torch.bfloat16, device=dev)
     hi = terms.data_ptr()
     _lib.check(H.bf16x_split_terms(x2, code, M * in_f, hi, hi + 2 * M * in_f, st), "bf16x_split_terms")

@@ -287,6 +287,18 @@ int bf16x_gemm_chunks(const void* x, int32_t x_dtype, int64_t M,
 int bf16x_split_terms(const void* x, int32_t x_dtype, int64_t n, uint16_t* hi, uint16_t* lo, bf16x_stream_t stream);
 int bf16x_add_terms(const float* a, const float* b, int64_t n, void* y, int32_t y_dtype, bf16x_stream_t stream);
 
+/* bf16x_gemm for fp16 / fp32 activations, both bf16 terms of x (hi and lo, as
+ * above) multiplied into one fp32 accumulator; y in x's type.  For the shapes
+ * where bf16x_gemm runs the grouped wave-specialised kernel at 2 M rows;
+ * bf16x_gemm_terms_workspace returns BF16X_ESHAPE for others.  x 4-byte
+ * aligned; workspace (16-byte aligned), plan and modes as in bf16x_gemm. */
+int64_t bf16x_gemm_terms_workspace(int64_t M, int64_t out_f, int64_t in_f);
+int bf16x_gemm_terms(const void* x, int32_t x_dtype, int64_t M, const int32_t* sign, int64_t n_sign,
+                     const int32_t* mant, int64_t n_mant, const int32_t* delta, int64_t n_delta,
+                     const uint8_t* emax, int64_t n_emax, const uint32_t* kp_off, const uint32_t* kp_ent,
+                     int64_t out_f, int64_t in_f, int32_t sub, int32_t mode, void* y, void* workspace,
+                     int64_t workspace_bytes, bf16x_stream_t stream);
+
 /* ========================================================================
  * GGUF half-block variant (bf16x_gguf_block.py, GGML_TYPE_BF16X): blocks of
  * 32 row-major weights, 46 bytes = [emax[2] | sign[4] | mant[28] |

@@ -41,16 +41,26 @@ def test_split_and_add_terms(bx, dt, n, off):  # noqa: F811
     assert same(y, (a + b).to(dt))
 
 
-# 2 M rows on each kernel of the dispatch: 2 (one row), 16 / 18, 64 / 66,
-# 128 / 130 and past 256; a row-offset view (contiguous, 2 bytes off 16)
+# 2 M rows on each kernel of the dispatch: 2 (one row), 16 / 18, 64; from 33
+# rows the kernel that takes both terms (tiles of 64 and 128 tokens, whole K
+# and split), except at in_f % 256 != 0; a row-offset view (contiguous, its
+# start aligned to one element only), which a 2-byte type splits first
 @pytest.mark.parametrize("dt", [torch.float16, torch.float32])
-@pytest.mark.parametrize("M", [1, 8, 9, 32, 33, 64, 65, 200])
-def test_gemm_terms(bx, dt, M):  # noqa: F811
-    out_f, in_f = 520, 2048
+@pytest.mark.parametrize("exact", [True, False])
+@pytest.mark.parametrize("M,out_f,in_f,split,off", [
+    (1, 520, 2048, -1, 1), (8, 520, 2048, -1, 0), (9, 520, 2048, -1, 1), (32, 520, 2048, -1, 0),
+    (33, 520, 2048, -1, 0), (33, 520, 2048, -1, 1), (64, 130, 1024, 1, 0), (65, 300, 1024, 3, 2),
+    (128, 128, 256, -1, 0), (129, 200, 768, -1, 0), (200, 520, 2048, -1, 0), (300, 96, 4096, 2, 0),
+    (100, 520, 2112, -1, 0)])
+def test_gemm_terms(bx, tune, dt, exact, M, out_f, in_f, split, off):  # noqa: F811
+    tune(gemm_ws_split=split)
     w = bits_tensor(dc.bench_weight_bits(out_f, in_f, seed=M))
     d = bx.bf16x_quantize(w.to(DEV))
-    plan = bx.build_plan_host(d, device=DEV)
-    x = torch.randn(M * in_f + 1, generator=torch.Generator().manual_seed(M)).to(dt).to(DEV)[1:].view(M, in_f)
+    plan = bx.build_plan_host(d, device=DEV) if exact else None
+    if not exact:
+        w = bits_tensor(dc.decode_saturated({k: (v.cpu().numpy() if isinstance(v, torch.Tensor) else v)
+                                             for k, v in d.items()}).reshape(out_f, in_f))
+    x = torch.randn(M * in_f + off, generator=torch.Generator().manual_seed(M)).to(dt).to(DEV)[off:].view(M, in_f)
     y = bx.bf16x_gemm(x, d["sign_packed"], d["mant_packed"], d["delta_packed"], d["emax"], out_f, in_f, plan=plan,
                       path="fused")
     assert y.dtype == dt and y.shape == (M, out_f)
