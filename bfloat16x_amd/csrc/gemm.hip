@@ -484,10 +484,10 @@ extern "C" int bf16x_gguf_kplan_build(const uint32_t* row_off, const uint32_t* e
 
 // wave-specialised kernel (gemm_ws.hip): M >= ws_rows()
 int64_t bf16x_gemm_ws_workspace(int64_t M, int64_t out_f, int64_t in_f, bool terms);
-int bf16x_gemm_ws_launch(const void* x, int32_t x_dtype, int64_t M, const uint32_t* s, const uint32_t* m, const uint32_t* d,
-                         const uint16_t* e, const uint8_t* blocks, const uint32_t* kp_off, const uint32_t* kp_ent,
-                         int64_t out_f, int64_t in_f, bool exact, bool yf32, void* y, void* workspace,
-                         int64_t workspace_bytes, hipStream_t st);
+int bf16x_gemm_ws_launch(const void* x, int32_t x_dtype, int64_t M, const uint32_t* s, const uint32_t* m,
+                         const uint32_t* d, const uint16_t* e, const uint8_t* blocks, const uint32_t* kp_off,
+                         const uint32_t* kp_ent, int64_t out_f, int64_t in_f, bool exact, bool yf32, void* y,
+                         void* workspace, int64_t workspace_bytes, hipStream_t st);
 
 // few-row kernel (gemm_skinny.hip): M <= skinny_rows()
 int bf16x_gemm_skinny_launch(const uint16_t* x, int64_t M, const uint32_t* s, const uint32_t* m, const uint32_t* d,
@@ -495,11 +495,11 @@ int bf16x_gemm_skinny_launch(const uint16_t* x, int64_t M, const uint32_t* s, co
                              int64_t in_f, bool exact, bool yf32, void* y, hipStream_t st);
 
 // few-row MFMA kernel (gemm_skinny2.hip): M <= skinny2_rows(), in_f % 128 == 0
-int64_t bf16x_gemm_skinny2_workspace(int64_t M, int64_t out_f, int64_t in_f);
+int64_t bf16x_gemm_skinny2_workspace(int64_t M, int64_t out_f, int64_t in_f, bool gg);
 int bf16x_gemm_skinny2_launch(const uint16_t* x, int64_t M, const uint32_t* s, const uint32_t* m,
-                              const uint32_t* d, const uint16_t* e, const uint32_t* kp_off, const uint32_t* kp_ent,
-                              int64_t out_f, int64_t in_f, bool exact, bool yf32, void* y, void* workspace,
-                              int64_t workspace_bytes, hipStream_t st);
+                              const uint32_t* d, const uint16_t* e, const uint8_t* blocks, const uint32_t* kp_off,
+                              const uint32_t* kp_ent, int64_t out_f, int64_t in_f, bool exact, bool yf32, void* y,
+                              void* workspace, int64_t workspace_bytes, hipStream_t st);
 
 namespace {
 
@@ -585,7 +585,7 @@ GemmShape gemm_shape(int64_t M, int64_t out_f, int64_t in_f) {
 
 extern "C" int64_t bf16x_gemm_workspace(int64_t M, int64_t out_f, int64_t in_f) {
   if (M <= 0 || out_f <= 0 || in_f < kBK) return 0;
-  if (use_skinny2(M, out_f, in_f)) return bf16x_gemm_skinny2_workspace(M, out_f, in_f);
+  if (use_skinny2(M, out_f, in_f)) return bf16x_gemm_skinny2_workspace(M, out_f, in_f, false);
   if (M <= skinny_rows()) return 0;
   if (use_ws(M, out_f, in_f)) return bf16x_gemm_ws_workspace(M, out_f, in_f, false);
   const GemmShape g = gemm_shape(M, out_f, in_f);
@@ -612,7 +612,7 @@ extern "C" int bf16x_gemm(const void* x, int32_t x_dtype, int64_t M, const int32
   hipStream_t st = (hipStream_t)stream;
   if (use_skinny2(M, out_f, in_f)) {
     rc = bf16x_gemm_skinny2_launch((const uint16_t*)x, M, (const uint32_t*)sign, (const uint32_t*)mant,
-                                   (const uint32_t*)delta, (const uint16_t*)emax, kp_off, kp_ent, out_f, in_f,
+                                   (const uint32_t*)delta, (const uint16_t*)emax, nullptr, kp_off, kp_ent, out_f, in_f,
                                    mode == BF16X_EXACT, y_dtype == BF16X_F32, y, workspace, workspace_bytes, st);
     return rc ? rc : launch_status();
   }

@@ -38,6 +38,7 @@
 #include <stdlib.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "../../include/bf16x_hip.h"
 #include "bf16x_device.h"
@@ -68,6 +69,10 @@ struct WAtom {
   uint32_t s, m[7], d[3];
   uint32_t ew;     // dword holding this atom's emax pair (and its neighbour's)
 };
+// a GGUF block as loaded: the 48 bytes from the dword at or below it
+struct WBlock {
+  u32x4 q0, q1, q2;
+};
 struct Bounds { uint32_t b0, e0, b1, e1; };
 struct Ents { uint32_t v[2]; };
 
@@ -77,12 +82,16 @@ struct Ents { uint32_t v[2]; };
 // line once for all of them (requests to a line already in flight are
 // merged) instead of once per step.  The KQ partial sums of a row group are
 // added in wave order at the end.
-template <int NC, int KQ, bool EXACT, bool PARTIAL, bool YF32>
+//
+// GG: W is GGUF half-blocks (`blocks`, 46 bytes per 32 elements; the dict
+// streams are unused), decoded with the zero marker (bf16x_gguf_block.py:76-87);
+// a quad of lanes reads 184 contiguous bytes of a row.
+template <bool GG, int NC, int KQ, bool EXACT, bool PARTIAL, bool YF32>
 __global__ __launch_bounds__(256 * KQ) void gemm_skinny2_kernel(
     const uint16_t* __restrict__ x, int64_t M, const uint32_t* __restrict__ sign,
     const uint32_t* __restrict__ mant, const uint32_t* __restrict__ delta, const uint16_t* __restrict__ emax2,
-    const uint32_t* __restrict__ kp_off, const uint32_t* __restrict__ kp_ent, int64_t out_f, int64_t in_f,
-    int sps, void* __restrict__ out) {
+    const uint8_t* __restrict__ blocks, const uint32_t* __restrict__ kp_off, const uint32_t* __restrict__ kp_ent,
+    int64_t out_f, int64_t in_f, int sps, void* __restrict__ out) {
   constexpr int D = KQ == 1 ? 4 : 2;               // workgroup steps of W atoms in flight (even)
   constexpr int NT = 256 * KQ;                     // threads
   constexpr int MP = NC * 16;                      // tokens padded to whole MFMA blocks
@@ -113,24 +122,45 @@ __global__ __launch_bounds__(256 * KQ) void gemm_skinny2_kernel(
   // ---- W atoms: lane -> (row n0w + rl, atom 4 s + ql); the step enters as a
   // uniform scalar offset
   const int64_t wrow = min(n0w + rl, out_f - 1);
-  const __amdgpu_buffer_rsrc_t rs_ = rsrc(sign, (uint64_t)out_f * P * 4);
-  const __amdgpu_buffer_rsrc_t rm_ = rsrc(mant, (uint64_t)out_f * P * 28);
-  const __amdgpu_buffer_rsrc_t rd_ = rsrc(delta, (uint64_t)out_f * P * 12);
-  const __amdgpu_buffer_rsrc_t re_ = rsrc(emax2, (uint64_t)out_f * P * 2);
-  const uint32_t av = (uint32_t)(wrow * P) + (uint32_t)ql;
-  const uint32_t vo_m = av * 28, vo_d = av * 12, vo_s = av * 4, vo_e = (av & ~1u) * 2;
-  const uint32_t esh = 16u * (av & 1u);            // P % 4 == 0: the parity of the atom index is step-invariant
-  auto load_w = [&](int m, WAtom& t) {
+  using WT = typename std::conditional<GG, WBlock, WAtom>::type;
+  __amdgpu_buffer_rsrc_t rs_, rm_, rd_, re_, rb_;
+  uint32_t vo_m = 0, vo_d = 0, vo_s = 0, vo_e = 0, vo_b = 0;
+  uint32_t esh;                                    // P % 4 == 0: the parity of the atom index is step-invariant
+  if constexpr (GG) {
+    // the tile's first block (64 rows of P % 4 == 0 blocks in) starts at a
+    // multiple of 4 bytes, and so does every step; the range is the rest of
+    // the blocks rounded up to 4 bytes, which the caller guarantees readable
+    const int64_t t0 = (int64_t)tile * kRowsBlock;
+    const uint32_t av = (uint32_t)((wrow - t0) * P) + (uint32_t)ql;
+    rb_ = rsrc(blocks + (uint64_t)t0 * P * 46, ((uint64_t)(out_f - t0) * P * 46 + 3) & ~3ull);
+    vo_b = (av * 46) & ~3u;
+    esh = 16u * (av & 1u);
+  } else {
+    const uint32_t av = (uint32_t)(wrow * P) + (uint32_t)ql;
+    rs_ = rsrc(sign, (uint64_t)out_f * P * 4);
+    rm_ = rsrc(mant, (uint64_t)out_f * P * 28);
+    rd_ = rsrc(delta, (uint64_t)out_f * P * 12);
+    re_ = rsrc(emax2, (uint64_t)out_f * P * 2);
+    vo_m = av * 28; vo_d = av * 12; vo_s = av * 4; vo_e = (av & ~1u) * 2;
+    esh = 16u * (av & 1u);
+  }
+  auto load_w = [&](int m, WT& t) {
     const uint32_t sa = 4u * (uint32_t)(s0 + wstep(m));
-    const u32x4 m03 = __builtin_amdgcn_raw_buffer_load_b128(rm_, (int)vo_m, (int)(sa * 28), 0);
-    const u32x3 m46 = __builtin_amdgcn_raw_buffer_load_b96(rm_, (int)(vo_m + 16), (int)(sa * 28), 0);
-    const u32x3 d02 = __builtin_amdgcn_raw_buffer_load_b96(rd_, (int)vo_d, (int)(sa * 12), 0);
-    t.s = __builtin_amdgcn_raw_buffer_load_b32(rs_, (int)vo_s, (int)(sa * 4), 0);
-    t.ew = __builtin_amdgcn_raw_buffer_load_b32(re_, (int)vo_e, (int)(sa * 2), 0);
-    const uint32_t c0 = m03.x, c1 = m03.y, c2 = m03.z, c3 = m03.w, c4 = m46.x, c5 = m46.y, c6 = m46.z;
-    t.m[0] = c0; t.m[1] = c1; t.m[2] = c2; t.m[3] = c3; t.m[4] = c4; t.m[5] = c5; t.m[6] = c6;
-    const uint32_t e0 = d02.x, e1 = d02.y, e2 = d02.z;
-    t.d[0] = e0; t.d[1] = e1; t.d[2] = e2;
+    if constexpr (GG) {
+      t.q0 = __builtin_amdgcn_raw_buffer_load_b128(rb_, (int)vo_b, (int)(sa * 46), 0);
+      t.q1 = __builtin_amdgcn_raw_buffer_load_b128(rb_, (int)(vo_b + 16), (int)(sa * 46), 0);
+      t.q2 = __builtin_amdgcn_raw_buffer_load_b128(rb_, (int)(vo_b + 32), (int)(sa * 46), 0);
+    } else {
+      const u32x4 m03 = __builtin_amdgcn_raw_buffer_load_b128(rm_, (int)vo_m, (int)(sa * 28), 0);
+      const u32x3 m46 = __builtin_amdgcn_raw_buffer_load_b96(rm_, (int)(vo_m + 16), (int)(sa * 28), 0);
+      const u32x3 d02 = __builtin_amdgcn_raw_buffer_load_b96(rd_, (int)vo_d, (int)(sa * 12), 0);
+      t.s = __builtin_amdgcn_raw_buffer_load_b32(rs_, (int)vo_s, (int)(sa * 4), 0);
+      t.ew = __builtin_amdgcn_raw_buffer_load_b32(re_, (int)vo_e, (int)(sa * 2), 0);
+      const uint32_t c0 = m03.x, c1 = m03.y, c2 = m03.z, c3 = m03.w, c4 = m46.x, c5 = m46.y, c6 = m46.z;
+      t.m[0] = c0; t.m[1] = c1; t.m[2] = c2; t.m[3] = c3; t.m[4] = c4; t.m[5] = c5; t.m[6] = c6;
+      const uint32_t e0 = d02.x, e1 = d02.y, e2 = d02.z;
+      t.d[0] = e0; t.d[1] = e1; t.d[2] = e2;
+    }
   };
 
   // ---- x tile of a workgroup step (KQ steps) in pair order: chunk c = i * NT
@@ -228,9 +258,11 @@ __global__ __launch_bounds__(256 * KQ) void gemm_skinny2_kernel(
   // m+D (into at); MFMAs from the LDS x tile of m (skipped for a step past the
   // split); x of m+1 (registers xs) to the other LDS buffer, then x of m+3
   // into xs; barrier.
-  auto step = [&](int m, WAtom& at, XRaw (&xs)[XI], Ents& ec, Ents& en, Bounds& bc, const Bounds& bn) {
+  auto step = [&](int m, WT& at, XRaw (&xs)[XI], Ents& ec, Ents& en, Bounds& bc, const Bounds& bn) {
     uint32_t w[16];
-    {
+    if constexpr (GG) {
+      decode_pairs<true>(gguf_atom(GgufRaw{at.q0, at.q1, at.q2, esh}), w);
+    } else {
       Atom t;
       t.s = at.s;
 #pragma unroll
@@ -292,7 +324,7 @@ __global__ __launch_bounds__(256 * KQ) void gemm_skinny2_kernel(
   // ---- prologue: x(0) to LDS; then the loads in flight at the loop entry in
   // the order steps -D .. -1 would have issued them: atoms 0 .. D-2, x 1,
   // entries 0, bounds 1, atoms D-1, x 2
-  WAtom A[D];
+  WT A[D];
   Bounds Bd[2] = {};
   Ents E[2] = {};
   XRaw X[2][XI];
@@ -400,8 +432,8 @@ struct Split {
 // does; 64 rows at 14336 x 4096: 47 us against 55 us with one wave per
 // row group).  The override BF16X_TUNE_SKINNY2_KQ = 1 or 2 replaces it.
 int nc_for(int64_t M) { return M <= 16 ? 1 : (M <= 32 ? 2 : 4); }
-int kq_for(int64_t M) {
-  const int64_t k = tuning(BF16X_TUNE_SKINNY2_KQ);
+int kq_for(int64_t M, bool gg) {
+  const int64_t k = gg ? -1 : tuning(BF16X_TUNE_SKINNY2_KQ);    // (the override is the dict kernels')
   if (k == 1) return 1;
   if (k == 2) return 2;
   return nc_for(M) <= 2 ? 4 : 2;
@@ -411,7 +443,7 @@ int kq_for(int64_t M) {
 // device, from the runtime's occupancy calculation (registers and LDS of the
 // compiled kernel); 3 (KQ = 1) or 1 (KQ = 2, 4) per CU on 256 CUs when there
 // is no device to ask.
-template <int NC, int KQ, bool EXACT>
+template <bool GG, int NC, int KQ, bool EXACT>
 int64_t resident_slots() {
   static int64_t cache[64];
   const int64_t dflt = KQ == 1 ? 768 : 256;
@@ -419,7 +451,7 @@ int64_t resident_slots() {
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return dflt;
   if (cache[dev] > 0) return cache[dev];
   int per_cu = 0, cus = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, gemm_skinny2_kernel<NC, KQ, EXACT, true, false>,
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, gemm_skinny2_kernel<GG, NC, KQ, EXACT, true, false>,
                                                    256 * KQ, 0) != hipSuccess ||
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || per_cu <= 0 || cus <= 0)
     return dflt;
@@ -427,31 +459,28 @@ int64_t resident_slots() {
   return cache[dev];
 }
 
-int64_t slots_for(int64_t M, bool exact) {
-  const int nc = nc_for(M), kq = kq_for(M);
-  if (kq == 4) {
-    if (nc == 1) return exact ? resident_slots<1, 4, true>() : resident_slots<1, 4, false>();
-    return exact ? resident_slots<2, 4, true>() : resident_slots<2, 4, false>();
-  }
-  if (kq == 2) {
-    if (nc == 4) return exact ? resident_slots<4, 2, true>() : resident_slots<4, 2, false>();
-    if (nc == 2) return exact ? resident_slots<2, 2, true>() : resident_slots<2, 2, false>();
-    return exact ? resident_slots<1, 2, true>() : resident_slots<1, 2, false>();
-  }
-  if (nc == 1) return exact ? resident_slots<1, 1, true>() : resident_slots<1, 1, false>();
-  if (nc == 2) return exact ? resident_slots<2, 1, true>() : resident_slots<2, 1, false>();
-  return exact ? resident_slots<4, 1, true>() : resident_slots<4, 1, false>();
+template <bool GG, int NC, int KQ>
+int64_t slots_of(bool exact) {
+  return exact ? resident_slots<GG, NC, KQ, true>() : resident_slots<GG, NC, KQ, false>();
+}
+int64_t slots_for(int64_t M, bool exact, bool gg) {
+  const int nc = nc_for(M), kq = kq_for(M, gg);
+  if (gg) return nc == 1 ? slots_of<true, 1, 4>(exact) : nc == 2 ? slots_of<true, 2, 4>(exact) : slots_of<true, 4, 2>(exact);
+  if (kq == 4) return nc == 1 ? slots_of<false, 1, 4>(exact) : slots_of<false, 2, 4>(exact);
+  if (kq == 2)
+    return nc == 4 ? slots_of<false, 4, 2>(exact) : nc == 2 ? slots_of<false, 2, 2>(exact) : slots_of<false, 1, 2>(exact);
+  return nc == 1 ? slots_of<false, 1, 1>(exact) : nc == 2 ? slots_of<false, 2, 1>(exact) : slots_of<false, 4, 1>(exact);
 }
 
 // K split: as many splits as keep the grid within one round of resident
 // workgroups, at least 2 workgroup steps each, steps per split a multiple of
 // KQ.  A second, partial round would cost a whole workgroup lifetime for a
 // few workgroups.
-Split skinny2_split(int64_t M, int64_t out_f, int64_t in_f, bool exact) {
+Split skinny2_split(int64_t M, int64_t out_f, int64_t in_f, bool exact, bool gg) {
   const int64_t tiles = (out_f + kRowsBlock - 1) / kRowsBlock;
   const int64_t S = in_f / kStep;
-  const int64_t kq = kq_for(M);
-  int64_t ks = slots_for(M, exact) / tiles;
+  const int64_t kq = kq_for(M, gg);
+  int64_t ks = slots_for(M, exact, gg) / tiles;
   ks = std::max<int64_t>(1, std::min<int64_t>(ks, S / (2 * kq)));
   if (const int64_t t = tuning(BF16X_TUNE_SKINNY2_SPLIT); t > 0) ks = std::min<int64_t>(t, S);
   Split sp;
@@ -467,23 +496,25 @@ Split skinny2_split(int64_t M, int64_t out_f, int64_t in_f, bool exact) {
 
 // Workspace of the few-row kernel: the fp32 partials of a K split (the larger
 // of the exact and the saturated kernel's split).
-int64_t bf16x_gemm_skinny2_workspace(int64_t M, int64_t out_f, int64_t in_f) {
+int64_t bf16x_gemm_skinny2_workspace(int64_t M, int64_t out_f, int64_t in_f, bool gg) {
   using namespace bf16x::skinny2;
-  const Split a = skinny2_split(M, out_f, in_f, true), b = skinny2_split(M, out_f, in_f, false);
+  const Split a = skinny2_split(M, out_f, in_f, true, gg), b = skinny2_split(M, out_f, in_f, false, gg);
   const Split sp = a.ks > b.ks ? a : b;
   return sp.ks > 1 ? (int64_t)sp.ks * M * out_f * 4 : 0;
 }
 
-// Shapes are validated by bf16x_gemm (in_f % 128 == 0 here, 32-bit offsets).
+// Shapes are validated by bf16x_gemm and bf16x_gguf_gemm (in_f % 128 == 0
+// here, 32-bit offsets).  GGUF: `blocks`, with the dict pointers null.
 int bf16x_gemm_skinny2_launch(const uint16_t* x, int64_t M, const uint32_t* s, const uint32_t* m,
-                              const uint32_t* d, const uint16_t* e, const uint32_t* kp_off, const uint32_t* kp_ent,
+                              const uint32_t* d, const uint16_t* e, const uint8_t* blocks, const uint32_t* kp_off, const uint32_t* kp_ent,
                               int64_t out_f, int64_t in_f, bool exact, bool yf32, void* y, void* workspace,
                               int64_t workspace_bytes, hipStream_t st) {
   using namespace bf16x::skinny2;
   if (M <= 0 || M > kMaxRows || in_f % kStep != 0) return BF16X_ESHAPE;
-  const Split sp = skinny2_split(M, out_f, in_f, exact);
+  const bool gg = blocks != nullptr;
+  const Split sp = skinny2_split(M, out_f, in_f, exact, gg);
   const bool partial = sp.ks > 1;
-  if (partial && (!workspace || workspace_bytes < bf16x_gemm_skinny2_workspace(M, out_f, in_f) ||
+  if (partial && (!workspace || workspace_bytes < bf16x_gemm_skinny2_workspace(M, out_f, in_f, gg) ||
                   ((uintptr_t)workspace & 3)))
     return BF16X_ECAPACITY;
   const int64_t tiles = (out_f + kRowsBlock - 1) / kRowsBlock;
@@ -491,35 +522,39 @@ int bf16x_gemm_skinny2_launch(const uint16_t* x, int64_t M, const uint32_t* s, c
   if (grid > INT32_MAX) return BF16X_ESHAPE;
   float* part = (float*)workspace;
   void* out = partial ? (void*)part : y;
-  const int nc = nc_for(M), kq = kq_for(M);
-#define BF16X_S2(NC_, KQ_, EX_, PA_, YF_)                                                                    \
-  hipLaunchKernelGGL((gemm_skinny2_kernel<NC_, KQ_, EX_, PA_, YF_>), dim3((unsigned)grid), dim3(256 * KQ_), 0, st, \
-                     x, M, s, m, d, e, kp_off, kp_ent, out_f, in_f, sp.sps, out)
-#define BF16X_S2_NC(NC_, KQ_)                                                                             \
+  const int nc = nc_for(M), kq = kq_for(M, gg);
+#define BF16X_S2(GG_, NC_, KQ_, EX_, PA_, YF_)                                                               \
+  hipLaunchKernelGGL((gemm_skinny2_kernel<GG_, NC_, KQ_, EX_, PA_, YF_>), dim3((unsigned)grid), dim3(256 * KQ_), \
+                     0, st, x, M, s, m, d, e, blocks, kp_off, kp_ent, out_f, in_f, sp.sps, out)
+#define BF16X_S2_NC(GG_, NC_, KQ_)                                                                        \
   do {                                                                                                   \
     if (partial) {                                                                                       \
-      if (exact) BF16X_S2(NC_, KQ_, true, true, false);                                                  \
-      else BF16X_S2(NC_, KQ_, false, true, false);                                                       \
+      if (exact) BF16X_S2(GG_, NC_, KQ_, true, true, false);                                                  \
+      else BF16X_S2(GG_, NC_, KQ_, false, true, false);                                                       \
     } else if (exact) {                                                                                  \
-      if (yf32) BF16X_S2(NC_, KQ_, true, false, true);                                                   \
-      else BF16X_S2(NC_, KQ_, true, false, false);                                                       \
+      if (yf32) BF16X_S2(GG_, NC_, KQ_, true, false, true);                                                   \
+      else BF16X_S2(GG_, NC_, KQ_, true, false, false);                                                       \
     } else {                                                                                             \
-      if (yf32) BF16X_S2(NC_, KQ_, false, false, true);                                                  \
-      else BF16X_S2(NC_, KQ_, false, false, false);                                                      \
+      if (yf32) BF16X_S2(GG_, NC_, KQ_, false, false, true);                                                  \
+      else BF16X_S2(GG_, NC_, KQ_, false, false, false);                                                      \
     }                                                                                                    \
   } while (0)
-  if (kq == 4) {
-    if (nc == 1) BF16X_S2_NC(1, 4);
-    else BF16X_S2_NC(2, 4);
+  if (gg) {
+    if (nc == 1) BF16X_S2_NC(true, 1, 4);
+    else if (nc == 2) BF16X_S2_NC(true, 2, 4);
+    else BF16X_S2_NC(true, 4, 2);
+  } else if (kq == 4) {
+    if (nc == 1) BF16X_S2_NC(false, 1, 4);
+    else BF16X_S2_NC(false, 2, 4);
   } else if (kq == 2) {
-    if (nc == 1) BF16X_S2_NC(1, 2);
-    else if (nc == 2) BF16X_S2_NC(2, 2);
-    else BF16X_S2_NC(4, 2);
+    if (nc == 1) BF16X_S2_NC(false, 1, 2);
+    else if (nc == 2) BF16X_S2_NC(false, 2, 2);
+    else BF16X_S2_NC(false, 4, 2);
   } else {
     switch (nc) {
-      case 1: BF16X_S2_NC(1, 1); break;
-      case 2: BF16X_S2_NC(2, 1); break;
-      default: BF16X_S2_NC(4, 1); break;
+      case 1: BF16X_S2_NC(false, 1, 1); break;
+      case 2: BF16X_S2_NC(false, 2, 1); break;
+      default: BF16X_S2_NC(false, 4, 1); break;
     }
   }
 #undef BF16X_S2_NC

@@ -624,18 +624,44 @@ extern "C" int bf16x_gguf_gemv_lossless(const void* x, int32_t x_dtype, const ui
 }
 
 // ---------------------------------------------------------------------------
-// Fused decode + GEMM over GGUF blocks: the wave-specialised kernel of
-// gemm_ws.hip with its block loader (46-byte blocks, zero-marker decode).
+// Fused decode + GEMM over GGUF blocks: the few-row kernel of gemm_skinny2.hip
+// and the wave-specialised kernel of gemm_ws.hip with their block loaders
+// (46-byte blocks, zero-marker decode).
 // The lossless table enters as the step-major plan of bf16x_gguf_kplan_build.
 // ---------------------------------------------------------------------------
 int64_t bf16x_gemm_ws_workspace(int64_t M, int64_t out_f, int64_t in_f, bool terms);
-int bf16x_gemm_ws_launch(const void* x, int32_t x_dtype, int64_t M, const uint32_t* s, const uint32_t* m, const uint32_t* d,
-                         const uint16_t* e, const uint8_t* blocks, const uint32_t* kp_off, const uint32_t* kp_ent,
-                         int64_t out_f, int64_t in_f, bool exact, bool yf32, void* y, void* workspace,
-                         int64_t workspace_bytes, hipStream_t st);
+int bf16x_gemm_ws_launch(const void* x, int32_t x_dtype, int64_t M, const uint32_t* s, const uint32_t* m,
+                         const uint32_t* d, const uint16_t* e, const uint8_t* blocks, const uint32_t* kp_off,
+                         const uint32_t* kp_ent, int64_t out_f, int64_t in_f, bool exact, bool yf32, void* y,
+                         void* workspace, int64_t workspace_bytes, hipStream_t st);
+
+int64_t bf16x_gemm_skinny2_workspace(int64_t M, int64_t out_f, int64_t in_f, bool gg);
+int bf16x_gemm_skinny2_launch(const uint16_t* x, int64_t M, const uint32_t* s, const uint32_t* m,
+                              const uint32_t* d, const uint16_t* e, const uint8_t* blocks, const uint32_t* kp_off,
+                              const uint32_t* kp_ent, int64_t out_f, int64_t in_f, bool exact, bool yf32, void* y,
+                              void* workspace, int64_t workspace_bytes, hipStream_t st);
+
+namespace {
+// Rows of x the 16x16x32 few-row kernel takes (gemm_skinny2.hip with the block
+// loader): up to 32, and up to 64 for weights below 2^25 elements.  The
+// wave-specialised kernel pays a fixed ~10 us more (operand-order pass, its
+// first tiles) and less per weight once there are four token blocks.  Measured,
+// lossless, few-row against 64-token tiles (us): 8192x8192 M = 2 / 16 / 32 / 64
+// 30.8 / 32.3 / 36.3 / 48.0 against 41.0 / 41.4 / 42.0 / 43.2; 4096x14336 28.7
+// / 30.0 / 34.0 / 43.4 against 39.0 / 39.5 / 40.1 / 41.1; 4096x4096 14.1 / 14.6
+// / 16.3 / 19.3 against 22.1 / 21.7 / 22.2 / 22.4; 1024x1024 9.2 / 9.3 / 10.8 /
+// 12.1 against 13.4 / 13.8 / 14.0 / 14.2.
+bool gguf_few_rows(int64_t M, int64_t out_f, int64_t in_f) {
+  if (in_f % 128 != 0) return false;
+  const int64_t t = tuning(BF16X_TUNE_GEMM_SKINNY2_MAX);
+  if (t >= 0) return M <= std::min<int64_t>(t, 64);
+  return M <= 32 || (M <= 64 && out_f * in_f < ((int64_t)1 << 25));
+}
+}  // namespace
 
 extern "C" int64_t bf16x_gguf_gemm_workspace(int64_t M, int64_t out_f, int64_t in_f) {
   if (M <= 0 || out_f <= 0 || in_f < 64 || (in_f % 64) != 0) return 0;
+  if (gguf_few_rows(M, out_f, in_f)) return bf16x_gemm_skinny2_workspace(M, out_f, in_f, true);
   return bf16x_gemm_ws_workspace(M, out_f, in_f, false);
 }
 
@@ -653,6 +679,12 @@ extern "C" int bf16x_gguf_gemm(const void* x, int32_t x_dtype, int64_t M, const 
     return BF16X_ESHAPE;
   if (!aligned16(x) || !aligned4(blocks) || !aligned4(y)) return BF16X_EARG;
   if (kp_off && (!aligned4(kp_off) || !aligned4(kp_ent))) return BF16X_EARG;
+  if (gguf_few_rows(M, out_f, in_f)) {
+    rc = bf16x_gemm_skinny2_launch((const uint16_t*)x, M, nullptr, nullptr, nullptr, nullptr, blocks, kp_off, kp_ent,
+                                   out_f, in_f, kp_off != nullptr, y_dtype == BF16X_F32, y, workspace,
+                                   workspace_bytes, (hipStream_t)stream);
+    return rc ? rc : launch_status();
+  }
   rc = bf16x_gemm_ws_launch(x, BF16X_BF16, M, nullptr, nullptr, nullptr, nullptr, blocks, kp_off, kp_ent, out_f,
                             in_f, kp_off != nullptr, y_dtype == BF16X_F32, y, workspace, workspace_bytes,
                             (hipStream_t)stream);

@@ -133,7 +133,28 @@ def test_gemm_fused_token_tiles(g, tune, kind, shape, M):
     blocks = g.device_blocks(packed, DEV)
     xm = torch.randn(M, shape[1], generator=torch.Generator().manual_seed(M)).to(torch.bfloat16)
     for bm in (64, 128, 256):
-        tune(gemm_ws_bm=bm)
+        tune(gemm_ws_bm=bm, gemm_skinny2_max=0)
         for ovf, ref in ((t, wb), (None, wnl)):
             y = g.gguf_gemm_fused(xm.to(DEV), blocks, *shape, out_dtype=torch.float32, ovf=ovf)
             check_tol(y.cpu().numpy(), xm.double().numpy() @ ref.T)
+
+
+# The few-row kernel (up to 32 rows; up to 64 when asked): 16-token blocks, the
+# widths its steps and splits leave ragged (one 128-column step, an odd
+# number, many), rows around a 16-row wave and a 64-row tile
+@pytest.mark.parametrize("kind", ["dense", "selftest"])
+@pytest.mark.parametrize("shape", [(15, 128), (64, 640), (130, 2048), (300, 1152)])
+@pytest.mark.parametrize("M", [2, 16, 17, 32, 33, 64])
+def test_gemm_few_rows(g, tune, kind, shape, M):
+    tune(gemm_skinny2_max=64)
+    w = weights(kind, shape, 12)
+    wb = go.bf16_bits_to_fp32(go.fp32_to_bf16_bits(w)).astype(np.float64).reshape(shape)
+    packed = g.quantize_blocks(w)
+    wnl = go.dequantize_blocks(packed).astype(np.float64).reshape(shape)
+    t = g.device_ovf(g.pack_ovf(w), packed, DEV)
+    blocks = g.device_blocks(packed, DEV)
+    xm = torch.randn(M, shape[1], generator=torch.Generator().manual_seed(M)).to(torch.bfloat16)
+    for ovf, ref in ((t, wb), (None, wnl)):
+        for dt in (torch.float32, torch.bfloat16):
+            y = g.gguf_gemm_fused(xm.to(DEV), blocks, *shape, out_dtype=dt, ovf=ovf)
+            check_tol(y.float().cpu().numpy(), xm.double().numpy() @ ref.T)
