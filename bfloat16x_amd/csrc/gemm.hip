@@ -369,80 +369,212 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(const float* __restric
 
 // ---------------------------------------------------------------------------
 // Step-major plan from the row plan (one tile per row, in_f <= 65536).  One
-// 64-lane block per 32-row group; lane r < 32 walks the entries of row
-// g*32 + r, which are sorted by column; lanes 0-15 and 16-31 make the runs of
-// the 16-row groups 2g and 2g + 1.  Pass 1 counts each (step, 16-row group)
-// run, a one-block scan turns counts into offsets, pass 2 writes the entries.
+// workgroup per 16-row group h: its rows' entries are one contiguous run of
+// the row plan, so they are read coalesced.  The count kernel makes the
+// histogram over the steps, a scan turns the counts into offsets, and the
+// fill kernel writes each entry at run offset + entries of the rows above in
+// that run (a row-by-step table in LDS, prefixed over the rows) + entries of
+// its own row and step before it.  Every first product with a weight waits for
+// this: 14336x4096 12 + 10 + 24 us, where one 64-lane workgroup per 32 rows
+// walking the steps, and a scan by one workgroup, took 119 + 101 + 151 (the
+// first product with new weights, 101 rows: 613 -> 120 us).
+// Entries of a row are strictly ascending in every plan the builders make; a
+// group where they are not (or whose offsets or columns are out of order or
+// range) takes the walk: lane r takes row r's entries step by step, stopping
+// at the first that is out of order.
 // GE: entries of the GGUF side table (column | bits << 16) instead of the row
 // plan's (column << 16 | bits).
 // ---------------------------------------------------------------------------
+template <bool GE>
+__device__ __forceinline__ uint32_t kplan_col(uint32_t e) { return GE ? e & 0xFFFFu : e >> 16; }
+template <bool GE>
+__device__ __forceinline__ uint32_t kplan_entry(int64_t row, uint32_t e) {
+  const uint32_t bits = GE ? e >> 16 : e & 0xFFFFu;
+  return ((uint32_t)(row & 255) << 22) | ((kplan_col<GE>(e) & 63u) << 16) | bits;
+}
+
+// wave 0: counts (FILL = false) or entries of group h, row by lane
 template <bool FILL, bool GE>
-__global__ __launch_bounds__(64) void kplan_pass_kernel(const uint32_t* __restrict__ tile_off,
-                                                        const uint32_t* __restrict__ tile_ent, int64_t out_f,
-                                                        int S, int G2, uint32_t* __restrict__ kp_off,
-                                                        uint32_t* __restrict__ kp_ent) {
-  const int g = blockIdx.x, lane = threadIdx.x;
-  const int h = 2 * g + (lane >= 16 ? 1 : 0);    // 16-row group of this lane's row
-  const int64_t row = (int64_t)g * kGroupRows + lane;
-  const bool live = lane < kGroupRows && row < out_f;
+__device__ void kplan_walk(const uint32_t* __restrict__ tile_off, const uint32_t* __restrict__ tile_ent,
+                           int64_t out_f, int S, int G2, int h, uint32_t* __restrict__ kp_off,
+                           uint32_t* __restrict__ kp_ent) {
+  const int lane = threadIdx.x;
+  const int64_t row = (int64_t)h * 16 + lane;
+  const bool live = lane < 16 && row < out_f;
   uint32_t p = live ? tile_off[row] : 0, pe = live ? tile_off[row + 1] : 0;
   for (int s = 0; s < S; ++s) {
     uint32_t c = 0;
-    // column >> 6 == s
-    while (p + c < pe && ((GE ? tile_ent[p + c] & 0xFFFFu : tile_ent[p + c] >> 16) >> 6) == (uint32_t)s) ++c;
-    uint32_t incl = c;                   // inclusive prefix over the lanes
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const uint32_t v = __shfl_up(incl, o);
-      if (lane >= o) incl += v;
-    }
-    const uint32_t lo = __shfl(incl, 15);  // entries of the first 16-row group
-    const uint32_t all = __shfl(incl, 63);
+    while (p + c < pe && (kplan_col<GE>(tile_ent[p + c]) >> 6) == (uint32_t)s) ++c;
+    uint32_t all;
+    const uint32_t before = wave_prefix(c, lane, all);
     if constexpr (!FILL) {
-      if (lane == 0) {
-        kp_off[(int64_t)s * G2 + 2 * g] = lo;
-        kp_off[(int64_t)s * G2 + 2 * g + 1] = all - lo;
-      }
+      if (lane == 0) kp_off[(int64_t)s * G2 + h] = all;
     } else {
-      const uint32_t base = kp_off[(int64_t)s * G2 + h] + (lane >= 16 ? incl - lo : incl) - c;
-      for (uint32_t i = 0; i < c; ++i) {
-        const uint32_t e = tile_ent[p + i];
-        const uint32_t col = GE ? e & 0xFFFFu : e >> 16, bits = GE ? e >> 16 : e & 0xFFFFu;
-        kp_ent[base + i] = ((uint32_t)(row & 255) << 22) | ((col & 63u) << 16) | bits;
-      }
+      const uint32_t base = kp_off[(int64_t)s * G2 + h] + before;
+      for (uint32_t i = 0; i < c; ++i) kp_ent[base + i] = kplan_entry<GE>(row, tile_ent[p + i]);
     }
     p += c;
   }
 }
 
-// exclusive scan of a[0..n) in place, a[n] = total (one block)
-__global__ __launch_bounds__(1024) void kplan_scan_kernel(uint32_t* __restrict__ a, int64_t n) {
-  __shared__ uint32_t part[1024];
-  const int t = threadIdx.x;
-  const int64_t chunk = (n + 1023) / 1024;
-  const int64_t b = min((int64_t)t * chunk, n), e = min(b + chunk, n);
-  uint32_t s = 0;
-  for (int64_t i = b; i < e; ++i) s += a[i];
-  part[t] = s;
+// offsets of the group's rows to `off` (17); whether its entries are strictly
+// ascending within rows, in range, and its offsets ascending.  All threads.
+template <bool GE>
+__device__ bool kplan_group(const uint32_t* __restrict__ tile_off, const uint32_t* __restrict__ tile_ent,
+                            int64_t out_f, int S, int h, uint32_t* off, int* bad) {
+  const int tid = threadIdx.x;
+  if (tid == 0) *bad = 0;
+  if (tid < 17) off[tid] = tile_off[min((int64_t)h * 16 + tid, out_f)];
   __syncthreads();
-  for (int o = 1; o < 1024; o <<= 1) {
-    const uint32_t v = t >= o ? part[t - o] : 0u;
-    __syncthreads();
-    part[t] += v;
-    __syncthreads();
+  bool wrong = tid < 16 && off[tid] > off[tid + 1];
+  const uint32_t e0 = off[0], e1 = off[16];
+  for (uint32_t j = e0 + tid; j < e1 && j >= e0; j += 256) {
+    const uint32_t c = kplan_col<GE>(tile_ent[j]);
+    wrong |= (c >> 6) >= (uint32_t)S;
+    if (j > e0 && c <= kplan_col<GE>(tile_ent[j - 1])) {      // fine only where a row starts
+      bool start = false;
+#pragma unroll
+      for (int r = 1; r < 16; ++r) start |= off[r] == j;
+      wrong |= !start;
+    }
   }
-  uint32_t run = part[t] - s;
-  for (int64_t i = b; i < e; ++i) {
-    const uint32_t v = a[i];
-    a[i] = run;
-    run += v;
-  }
-  if (t == 1023) a[n] = part[1023];
+  if (wrong) *bad = 1;
+  __syncthreads();
+  return *bad == 0;
 }
 
-// Exclusive scan of a[0..n) in place on `st`, a[n] = the total (one block).
+template <bool GE>
+__global__ __launch_bounds__(256) void kplan_count_kernel(const uint32_t* __restrict__ tile_off,
+                                                          const uint32_t* __restrict__ tile_ent, int64_t out_f,
+                                                          int S, int G2, uint32_t* __restrict__ kp_off) {
+  extern __shared__ uint32_t cnt[];                    // [S]
+  __shared__ uint32_t off[17];
+  __shared__ int bad;
+  const int h = blockIdx.x, tid = threadIdx.x;
+  for (int s = tid; s < S; s += 256) cnt[s] = 0;
+  if (!kplan_group<GE>(tile_off, tile_ent, out_f, S, h, off, &bad)) {
+    if (tid < 64) kplan_walk<false, GE>(tile_off, tile_ent, out_f, S, G2, h, kp_off, nullptr);
+    return;
+  }
+  for (uint32_t j = off[0] + tid; j < off[16]; j += 256) atomicAdd(&cnt[kplan_col<GE>(tile_ent[j]) >> 6], 1u);
+  __syncthreads();
+  for (int s = tid; s < S; s += 256) kp_off[(int64_t)s * G2 + h] = cnt[s];
+}
+
+template <bool GE>
+__global__ __launch_bounds__(256) void kplan_fill_kernel(const uint32_t* __restrict__ tile_off,
+                                                         const uint32_t* __restrict__ tile_ent, int64_t out_f, int S,
+                                                         int G2, uint32_t* __restrict__ kp_off,
+                                                         uint32_t* __restrict__ kp_ent) {
+  // [16 rows][ceil(S / 2)] of two 16-bit counts: at most 64 entries per row
+  // and step, 1024 per run
+  extern __shared__ uint32_t cnt[];
+  __shared__ uint32_t off[17];
+  __shared__ int bad;
+  const int h = blockIdx.x, tid = threadIdx.x, W = (S + 1) / 2;
+  for (int i = tid; i < 16 * W; i += 256) cnt[i] = 0;
+  if (!kplan_group<GE>(tile_off, tile_ent, out_f, S, h, off, &bad)) {
+    if (tid < 64) kplan_walk<true, GE>(tile_off, tile_ent, out_f, S, G2, h, kp_off, kp_ent);
+    return;
+  }
+  auto row_of = [&](uint32_t j) {                      // last row starting at or before j
+    int r = 0;
+#pragma unroll
+    for (int b = 8; b; b >>= 1) r += off[r + b] <= j ? b : 0;
+    return r;
+  };
+  const uint32_t e0 = off[0], e1 = off[16];
+  for (uint32_t j = e0 + tid; j < e1; j += 256) {
+    const uint32_t s = kplan_col<GE>(tile_ent[j]) >> 6;
+    atomicAdd(&cnt[row_of(j) * W + (s >> 1)], 1u << (16 * (s & 1)));
+  }
+  __syncthreads();
+  for (int w = tid; w < W; w += 256) {
+    uint32_t run = 0;
+    for (int r = 0; r < 16; ++r) {
+      const uint32_t c = cnt[r * W + w];
+      cnt[r * W + w] = run;
+      run += c;                                        // both halves, each at most 1024
+    }
+  }
+  __syncthreads();
+  for (uint32_t j = e0 + tid; j < e1; j += 256) {
+    const uint32_t e = tile_ent[j], s = kplan_col<GE>(e) >> 6;
+    const int r = row_of(j);
+    uint32_t k = 0;                                    // entries of this row and step before it (< 64)
+    while (j - k > off[r] && (kplan_col<GE>(tile_ent[j - k - 1]) >> 6) == s) ++k;
+    const uint32_t above = (cnt[r * W + (s >> 1)] >> (16 * (s & 1))) & 0xFFFFu;
+    kp_ent[kp_off[(int64_t)s * G2 + h] + above + k] = kplan_entry<GE>((int64_t)h * 16 + r, e);
+  }
+}
+
+// Exclusive scan of a[0..n) in place, a[n] = the total, in tiles of kScanTile:
+// within the tiles (a tile's first element, whose exclusive sum is 0, holds
+// its total instead), over the tiles' first elements by one workgroup, and the
+// tiles' offsets (now their first elements) added to the rest of each.
+constexpr int kScanTile = 4096;
+
+__global__ __launch_bounds__(1024) void scan_tiles_kernel(uint32_t* __restrict__ a, int64_t n) {
+  __shared__ uint32_t part[16];
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int64_t i0 = (int64_t)blockIdx.x * kScanTile + 4 * tid;
+  uint32_t v[4], own = 0, total;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    v[k] = i0 + k < n ? a[i0 + k] : 0u;
+    own += v[k];
+  }
+  uint32_t at = wave_prefix(own, lane, total);
+  if (lane == 0) part[wv] = total;
+  __syncthreads();
+  uint32_t all = 0;
+  for (int k = 0; k < 16; ++k) {
+    if (k < wv) at += part[k];
+    all += part[k];
+  }
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    if (i0 + k < n) a[i0 + k] = tid == 0 && k == 0 ? all : at;
+    at += v[k];
+  }
+}
+
+__global__ __launch_bounds__(1024) void scan_firsts_kernel(uint32_t* __restrict__ a, int64_t n, int64_t tiles) {
+  __shared__ uint32_t part[16];
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  uint32_t carry = 0;
+  for (int64_t t0 = 0; t0 < tiles; t0 += 1024) {
+    const int64_t t = t0 + tid;
+    const uint32_t v = t < tiles ? a[t * kScanTile] : 0u;
+    uint32_t total;
+    uint32_t at = carry + wave_prefix(v, lane, total);
+    if (lane == 0) part[wv] = total;
+    __syncthreads();
+    for (int k = 0; k < 16; ++k) {
+      if (k < wv) at += part[k];
+      carry += part[k];
+    }
+    if (t < tiles) a[t * kScanTile] = at;
+    __syncthreads();
+  }
+  if (tid == 0) a[n] = carry;
+}
+
+__global__ __launch_bounds__(1024) void scan_add_kernel(uint32_t* __restrict__ a, int64_t n) {
+  const int64_t b = (int64_t)(blockIdx.x + 1) * kScanTile;      // (the first tile's offset is 0)
+  const uint32_t base = a[b];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int64_t i = b + k * 1024 + threadIdx.x;
+    if (i > b && i < n) a[i] += base;
+  }
+}
+
 void scan_offsets(uint32_t* a, int64_t n, hipStream_t st) {
-  hipLaunchKernelGGL(kplan_scan_kernel, dim3(1), dim3(1024), 0, st, a, n);
+  const int64_t tiles = (n + kScanTile - 1) / kScanTile;
+  if (tiles > 0) hipLaunchKernelGGL(scan_tiles_kernel, dim3((unsigned)tiles), dim3(1024), 0, st, a, n);
+  hipLaunchKernelGGL(scan_firsts_kernel, dim3(1), dim3(1024), 0, st, a, n, tiles);
+  if (tiles > 1) hipLaunchKernelGGL(scan_add_kernel, dim3((unsigned)(tiles - 1)), dim3(1024), 0, st, a, n);
 }
 
 }  // namespace bf16x
@@ -463,11 +595,11 @@ int kplan_build(const uint32_t* tile_off, const uint32_t* tile_ent, int64_t out_
   const int64_t S = in_f / kBK, G = (out_f + kGroupRows - 1) / kGroupRows, G2 = 2 * G;
   if (G2 > INT32_MAX || S * G2 + 1 > (int64_t)INT32_MAX) return BF16X_ESHAPE;
   hipStream_t st = (hipStream_t)stream;
-  hipLaunchKernelGGL((kplan_pass_kernel<false, GE>), dim3((unsigned)G), dim3(64), 0, st, tile_off, tile_ent, out_f,
-                     (int)S, (int)G2, kp_off, kp_ent);
+  hipLaunchKernelGGL(kplan_count_kernel<GE>, dim3((unsigned)G2), dim3(256), S * 4, st, tile_off, tile_ent, out_f,
+                     (int)S, (int)G2, kp_off);
   scan_offsets(kp_off, S * G2, st);
-  hipLaunchKernelGGL((kplan_pass_kernel<true, GE>), dim3((unsigned)G), dim3(64), 0, st, tile_off, tile_ent, out_f,
-                     (int)S, (int)G2, kp_off, kp_ent);
+  hipLaunchKernelGGL(kplan_fill_kernel<GE>, dim3((unsigned)G2), dim3(256), 16 * ((S + 1) / 2) * 4, st, tile_off,
+                     tile_ent, out_f, (int)S, (int)G2, kp_off, kp_ent);
   return launch_status();
 }
 }  // namespace
