@@ -66,6 +66,7 @@ namespace {
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kStep = 64;              // K columns per step
 constexpr int kRowB = 128;             // bytes of one LDS tile row (64 bf16)
@@ -859,73 +860,65 @@ void gemm_ws4_kernel(
 // is 1 KB at ((T * S + s) * 4 + q) * 1024, lane l = lr + 32 h holding row
 // 32 T + lr, columns 64 s + 32 h + {4q, 16+4q, 4q+1, 17+4q, .., 4q+3, 19+4q}
 // (the MFMA A operand of the fused kernels, in the K order of the W tile).
-// Rows past M (up to the 32-row boundary) are zeros.  One thread per
-// (T, s, l): it reads the 32 contiguous columns of its row (lanes l and l + 32
-// take the two halves of a 64-column row segment) and writes its 16 bytes of
-// each of the 4 k-quarters (each a contiguous 1 KB per wave).  XT fp16 or
-// fp32: two such matrices, hi = bf16(x) and, behind it, lo = bf16(x - hi).
-__device__ __forceinline__ void xo_store(const uint32_t (&w)[16], u32x4* __restrict__ xo, int64_t ts, int l) {
-  // quarter q: columns 4q .. 4q+3 (words 2q, 2q+1) and 16+4q .. 19+4q (words 8+2q, 9+2q)
-#pragma unroll
-  for (int q = 0; q < 4; ++q)
-    xo[(ts * 4 + q) * 64 + l] = u32x4{perm(w[8 + 2 * q], w[2 * q], 0x05040100u),
-                                      perm(w[8 + 2 * q], w[2 * q], 0x07060302u),
-                                      perm(w[9 + 2 * q], w[2 * q + 1], 0x05040100u),
-                                      perm(w[9 + 2 * q], w[2 * q + 1], 0x07060302u)};
+// Rows past M (up to the 32-row boundary) are zeros.  XT fp16 or fp32: two
+// such matrices, hi = bf16(x) and, behind it, lo = bf16(x - hi).  One thread
+// per 16-byte chunk (T, s, q, l): it reads the chunk's two runs of 4 columns
+// and writes it (1 KB contiguous per wave; the four waves of a workgroup take
+// the quarters of one (T, s), so a row's lines are shared in the L1).  At tens
+// of rows the pass is a launch and one memory round trip: with a thread per
+// row segment of 32 columns (a quarter of the threads, four chunks each)
+// 64x4096 fp16
+// took 5.2 us (3.0 here), 101x4096 bf16 4.0 (2.6), 512x4096 5.5 (4.4).
+__device__ __forceinline__ u32x4 xo_chunk(u32x2 a, u32x2 b) {
+  const uint32_t a0 = a.x, a1 = a.y, b0 = b.x, b1 = b.y;      // columns 4q .. 4q+3 and 16+4q .. 19+4q
+  return u32x4{perm(b0, a0, 0x05040100u), perm(b0, a0, 0x07060302u), perm(b1, a1, 0x05040100u),
+               perm(b1, a1, 0x07060302u)};
 }
 template <int XT>
 __global__ __launch_bounds__(256) void x_op_kernel(const void* __restrict__ x, int64_t M, int64_t in_f,
-                                                   int64_t units, u32x4* __restrict__ xo) {
-  const int64_t S = in_f / 64;
-  for (int64_t u = (int64_t)blockIdx.x * 256 + threadIdx.x; u < units; u += (int64_t)gridDim.x * 256) {
-    const int l = (int)(u & 63);
-    const int64_t ts = u >> 6, T = ts / S, s = ts - T * S;
-    const int64_t row = T * 32 + (l & 31);
-    const int64_t e0 = row * in_f + s * 64 + (l >> 5) * 32;
-    uint32_t w[16] = {0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u};
-    if constexpr (XT == BF16X_BF16) {
-      if (row < M) {
-        const u32x4a* src = (const u32x4a*)((const uint16_t*)x + e0);
+                                                   int64_t chunks, u32x4* __restrict__ xo) {
+  const uint32_t S = (uint32_t)(in_f / 64);      // (chunks < 2^28: x stays below 4 GiB)
+  for (int64_t u = (int64_t)blockIdx.x * 256 + threadIdx.x; u < chunks; u += (int64_t)gridDim.x * 256) {
+    const int l = (int)(u & 63), q = (int)(u >> 6) & 3;
+    const uint32_t ts = (uint32_t)(u >> 8), T = ts / S, s = ts - T * S;
+    const int64_t row = (int64_t)T * 32 + (l & 31);
+    const int64_t e0 = row * in_f + s * 64 + (l >> 5) * 32 + 4 * q;
+    u32x2 h[2] = {u32x2{0u, 0u}, u32x2{0u, 0u}}, r[2] = {u32x2{0u, 0u}, u32x2{0u, 0u}};
+    if (row < M) {
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          const u32x4a v = src[c];
-          const uint32_t v0 = v.x, v1 = v.y, v2 = v.z, v3 = v.w;
-          w[4 * c] = v0; w[4 * c + 1] = v1; w[4 * c + 2] = v2; w[4 * c + 3] = v3;
-        }
-      }
-      xo_store(w, xo, ts, l);
-    } else {
-      uint32_t lo[16] = {0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u};
-      if (row < M) {
-#pragma unroll
-        for (int k = 0; k < 16; ++k) {
-          float f[2];
+      for (int i = 0; i < 2; ++i) {
+        const int64_t e = e0 + 16 * i;
+        if constexpr (XT == BF16X_BF16) {
+          const u32x2a v = *(const u32x2a*)((const uint16_t*)x + e);
+          const uint32_t v0 = v.x, v1 = v.y;
+          h[i] = u32x2{v0, v1};
+        } else {
+          float f[4];
           if constexpr (XT == BF16X_F16) {
-            const uint32_t v = ((const u32x4a*)((const _Float16*)x + e0))[k >> 2][k & 3];
-            typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-            f16x2 h;
-            __builtin_memcpy(&h, &v, 4);
-            f[0] = (float)h.x;
-            f[1] = (float)h.y;
-          } else {
-            const u32x4a v = ((const u32x4a*)((const float*)x + e0))[k >> 1];
-            const uint32_t a = k & 1 ? v.z : v.x, b = k & 1 ? v.w : v.y;
-            f[0] = __uint_as_float(a);
-            f[1] = __uint_as_float(b);
-          }
-          uint32_t h[2], r[2];
+            const u32x2a v = *(const u32x2a*)((const _Float16*)x + e);
+            const uint32_t w[2] = {v.x, v.y};
+            _Float16 t[4];
+            __builtin_memcpy(t, w, 8);
 #pragma unroll
-          for (int i = 0; i < 2; ++i) {
-            h[i] = f32_to_bf16_rne(f[i]);
-            r[i] = f32_to_bf16_rne(f[i] - __uint_as_float(h[i] << 16));
+            for (int k = 0; k < 4; ++k) f[k] = (float)t[k];
+          } else {
+            const u32x4a v = *(const u32x4a*)((const float*)x + e);
+            const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+            __builtin_memcpy(f, w, 16);
           }
-          w[k] = h[0] | (h[1] << 16);
-          lo[k] = r[0] | (r[1] << 16);
+          uint32_t hi[4], lo[4];
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            hi[k] = f32_to_bf16_rne(f[k]);
+            lo[k] = f32_to_bf16_rne(f[k] - __uint_as_float(hi[k] << 16));
+          }
+          h[i] = u32x2{hi[0] | (hi[1] << 16), hi[2] | (hi[3] << 16)};
+          r[i] = u32x2{lo[0] | (lo[1] << 16), lo[2] | (lo[3] << 16)};
         }
       }
-      xo_store(w, xo, ts, l);
-      xo_store(lo, xo + units * 4, ts, l);
     }
+    xo[u] = xo_chunk(h[0], h[1]);
+    if constexpr (XT != BF16X_BF16) xo[u + chunks] = xo_chunk(r[0], r[1]);
   }
 }
 
@@ -939,14 +932,13 @@ __global__ __launch_bounds__(256) void ws_tile_reduce_kernel(const float* __rest
   // four consecutive columns of one tile row per thread (kBN % 4 == 0): 16-byte
   // partial loads, an 8-byte (bf16) or 16-byte (fp32) store when the row's
   // four outputs are in range and aligned (yal: y is 16-byte aligned)
-  const int64_t tsz = (int64_t)g.bm * kBN;
-  const int64_t count = (int64_t)g.ltiles * tsz;
+  // (at most resident blocks x 256 x 128 elements: 32-bit indexes)
+  const uint32_t tsz = (uint32_t)(g.bm * kBN), count = (uint32_t)g.ltiles * tsz, mt = (uint32_t)g.mtiles;
   typedef float f32x4v __attribute__((ext_vector_type(4)));
-  for (int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4; i < count; i += (int64_t)gridDim.x * 256 * 4) {
-    const int lt = (int)(i / tsz), e = (int)(i % tsz);
-    const int tile = g.full + lt;
-    const int64_t row = (int64_t)(tile % g.mtiles) * g.bm + e / kBN;
-    const int64_t col = (int64_t)(tile / g.mtiles) * kBN + e % kBN;
+  for (uint32_t i = (blockIdx.x * 256 + threadIdx.x) * 4; i < count; i += gridDim.x * 256 * 4) {
+    const uint32_t lt = i / tsz, e = i - lt * tsz, tile = (uint32_t)g.full + lt;
+    const int64_t row = (int64_t)(tile % mt) * g.bm + e / kBN;
+    const int64_t col = (int64_t)(tile / mt) * kBN + e % kBN;
     if (row >= M || col >= out_f) continue;
     f32x4v s = *(const f32x4v*)(part + i);
     for (int k = 1; k < nsplit; ++k) s += *(const f32x4v*)(part + (int64_t)k * count + i);
@@ -1026,7 +1018,8 @@ WsShape ws_shape(int64_t M, int64_t out_f, int64_t in_f, bool terms = false) {
   WsShape w;
   w.grouped = ws_grouped(in_f);
   const int64_t forced_c = tuning(BF16X_TUNE_GEMM_WS_RESIDENT);
-  const int64_t C = forced_c > 0 ? forced_c : ws_resident();
+  // (the reduction indexes the split tiles' elements in 32 bits)
+  const int64_t C = forced_c > 0 ? std::min<int64_t>(forced_c, 32768) : ws_resident();
   const int64_t nt = (out_f + kBN - 1) / kBN;
   const int64_t bm = w.grouped ? ws_tile_rows(M, nt, C, terms) : kBM;
   const int64_t mt = (M + bm - 1) / bm;
@@ -1035,7 +1028,7 @@ WsShape ws_shape(int64_t M, int64_t out_f, int64_t in_f, bool terms = false) {
   const int64_t max_split = std::max<int64_t>(1, std::min<int64_t>(16, w.grouped ? units : units / 4));
   int64_t f = tiles % C, s = f ? std::min<int64_t>(C / f, max_split) : 1;
   const int64_t forced = tuning(BF16X_TUNE_GEMM_WS_SPLIT);
-  if (forced > 0) {
+  if (forced > 0 && tiles <= 32768) {
     f = tiles;
     s = std::min<int64_t>(forced, w.grouped ? units : S);
   }
@@ -1085,14 +1078,14 @@ int bf16x_gemm_ws_launch(const void* x, int32_t x_dtype, int64_t M, const uint32
     return BF16X_ECAPACITY;
   if (xop >= (int64_t)0xFFFFFFFF) return BF16X_ESHAPE;
   if (w.grid > INT32_MAX) return BF16X_ESHAPE;
-  const int64_t units = xop / 64;   // (32-row tile, step, lane): 4 chunks of 16 bytes each
-  const dim3 xg((unsigned)std::min<int64_t>((units + 255) / 256, 8192));
+  const int64_t chunks = xop / 16;
+  const dim3 xg((unsigned)std::min<int64_t>((chunks + 255) / 256, 16384));
   if (x_dtype == BF16X_F16)
-    hipLaunchKernelGGL(x_op_kernel<BF16X_F16>, xg, dim3(256), 0, st, x, M, in_f, units, (u32x4*)workspace);
+    hipLaunchKernelGGL(x_op_kernel<BF16X_F16>, xg, dim3(256), 0, st, x, M, in_f, chunks, (u32x4*)workspace);
   else if (x_dtype == BF16X_F32)
-    hipLaunchKernelGGL(x_op_kernel<BF16X_F32>, xg, dim3(256), 0, st, x, M, in_f, units, (u32x4*)workspace);
+    hipLaunchKernelGGL(x_op_kernel<BF16X_F32>, xg, dim3(256), 0, st, x, M, in_f, chunks, (u32x4*)workspace);
   else
-    hipLaunchKernelGGL(x_op_kernel<BF16X_BF16>, xg, dim3(256), 0, st, x, M, in_f, units, (u32x4*)workspace);
+    hipLaunchKernelGGL(x_op_kernel<BF16X_BF16>, xg, dim3(256), 0, st, x, M, in_f, chunks, (u32x4*)workspace);
   const uint16_t* xo = (const uint16_t*)workspace;
   float* part = (float*)((uint8_t*)workspace + xop * (terms ? 2 : 1));
   const dim3 grid((unsigned)w.grid);
