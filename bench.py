@@ -112,6 +112,10 @@ def gemm_kernel_name(M: int, out_f: int, in_f: int) -> str:
         return "gemm_rows_kernel (rows streamed as in the GEMV, 16x16x32 MFMA)"
     if ops._use_chunks(M, out_f, in_f, torch.device("cuda:0")):
         return "gemm_chunks_kernel (rows streamed in column chunks, 16x16x32 MFMA)"
+    cus = torch.cuda.get_device_properties("cuda:0").multi_processor_count
+    steps = -(-(-(-out_f // 16)) // cus) * -(-(in_f // 128) // 16)
+    if M <= 16 and in_f % 128 == 0 and steps <= 4 and steps * M <= 32:
+        return "gemm_stream_kernel (streaming, 16x16x32 MFMA)"
     ws4 = in_f % 256 == 0 and (M > 64 or (M > 32 and out_f * in_f >= 1 << 25))
     if M <= 64 and in_f % 128 == 0 and not ws4:
         return "gemm_skinny2_kernel (16x16x32 MFMA, few rows)"

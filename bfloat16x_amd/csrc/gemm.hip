@@ -621,10 +621,18 @@ int bf16x_gemm_ws_launch(const void* x, int32_t x_dtype, int64_t M, const uint32
                          const uint32_t* kp_ent, int64_t out_f, int64_t in_f, bool exact, bool yf32, void* y,
                          void* workspace, int64_t workspace_bytes, hipStream_t st);
 
+bool bf16x_use_stream(int64_t M, int64_t out_f, int64_t in_f, bool gg);
+
 // few-row kernel (gemm_skinny.hip): M <= skinny_rows()
 int bf16x_gemm_skinny_launch(const uint16_t* x, int64_t M, const uint32_t* s, const uint32_t* m, const uint32_t* d,
                              const uint16_t* e, const uint32_t* kp_off, const uint32_t* kp_ent, int64_t out_f,
                              int64_t in_f, bool exact, bool yf32, void* y, hipStream_t st);
+
+// streaming few-row kernel (gemm_stream.hip): M <= 16, no workspace
+bool bf16x_gemm_stream_fits(int64_t M, int64_t out_f, int64_t in_f, bool gg);
+int bf16x_gemm_stream_launch(const uint16_t* x, int64_t M, const uint32_t* s, const uint32_t* m, const uint32_t* d,
+                             const uint16_t* e, const uint8_t* blocks, const uint32_t* kp_off, const uint32_t* kp_ent,
+                             int64_t out_f, int64_t in_f, bool exact, bool yf32, void* y, hipStream_t st);
 
 // few-row MFMA kernel (gemm_skinny2.hip): M <= skinny2_rows(), in_f % 128 == 0
 int64_t bf16x_gemm_skinny2_workspace(int64_t M, int64_t out_f, int64_t in_f, bool gg);
@@ -717,6 +725,7 @@ GemmShape gemm_shape(int64_t M, int64_t out_f, int64_t in_f) {
 
 extern "C" int64_t bf16x_gemm_workspace(int64_t M, int64_t out_f, int64_t in_f) {
   if (M <= 0 || out_f <= 0 || in_f < kBK) return 0;
+  if (bf16x_use_stream(M, out_f, in_f, false)) return 0;
   if (use_skinny2(M, out_f, in_f)) return bf16x_gemm_skinny2_workspace(M, out_f, in_f, false);
   if (M <= skinny_rows()) return 0;
   if (use_ws(M, out_f, in_f)) return bf16x_gemm_ws_workspace(M, out_f, in_f, false);
@@ -742,6 +751,10 @@ extern "C" int bf16x_gemm(const void* x, int32_t x_dtype, int64_t M, const int32
   if (!aligned4(sign) || !aligned4(mant) || !aligned4(delta) || !aligned2(emax) || !aligned16(x) || !aligned4(y))
     return BF16X_EARG;
   hipStream_t st = (hipStream_t)stream;
+  if (bf16x_use_stream(M, out_f, in_f, false))
+    return bf16x_gemm_stream_launch((const uint16_t*)x, M, (const uint32_t*)sign, (const uint32_t*)mant,
+                                    (const uint32_t*)delta, (const uint16_t*)emax, nullptr, kp_off, kp_ent, out_f,
+                                    in_f, mode == BF16X_EXACT, y_dtype == BF16X_F32, y, st);
   if (use_skinny2(M, out_f, in_f)) {
     rc = bf16x_gemm_skinny2_launch((const uint16_t*)x, M, (const uint32_t*)sign, (const uint32_t*)mant,
                                    (const uint32_t*)delta, (const uint16_t*)emax, nullptr, kp_off, kp_ent, out_f, in_f,

@@ -635,6 +635,12 @@ int bf16x_gemm_ws_launch(const void* x, int32_t x_dtype, int64_t M, const uint32
                          const uint32_t* kp_ent, int64_t out_f, int64_t in_f, bool exact, bool yf32, void* y,
                          void* workspace, int64_t workspace_bytes, hipStream_t st);
 
+// streaming few-row kernel (gemm_stream.hip): M <= 16, no workspace
+bool bf16x_gemm_stream_fits(int64_t M, int64_t out_f, int64_t in_f, bool gg);
+int bf16x_gemm_stream_launch(const uint16_t* x, int64_t M, const uint32_t* s, const uint32_t* m, const uint32_t* d,
+                             const uint16_t* e, const uint8_t* blocks, const uint32_t* kp_off, const uint32_t* kp_ent,
+                             int64_t out_f, int64_t in_f, bool exact, bool yf32, void* y, hipStream_t st);
+bool bf16x_use_stream(int64_t M, int64_t out_f, int64_t in_f, bool gg);
 int64_t bf16x_gemm_skinny2_workspace(int64_t M, int64_t out_f, int64_t in_f, bool gg);
 int bf16x_gemm_skinny2_launch(const uint16_t* x, int64_t M, const uint32_t* s, const uint32_t* m,
                               const uint32_t* d, const uint16_t* e, const uint8_t* blocks, const uint32_t* kp_off,
@@ -661,6 +667,7 @@ bool gguf_few_rows(int64_t M, int64_t out_f, int64_t in_f) {
 
 extern "C" int64_t bf16x_gguf_gemm_workspace(int64_t M, int64_t out_f, int64_t in_f) {
   if (M <= 0 || out_f <= 0 || in_f < 64 || (in_f % 64) != 0) return 0;
+  if (bf16x_use_stream(M, out_f, in_f, true)) return 0;
   if (gguf_few_rows(M, out_f, in_f)) return bf16x_gemm_skinny2_workspace(M, out_f, in_f, true);
   return bf16x_gemm_ws_workspace(M, out_f, in_f, false);
 }
@@ -679,6 +686,9 @@ extern "C" int bf16x_gguf_gemm(const void* x, int32_t x_dtype, int64_t M, const 
     return BF16X_ESHAPE;
   if (!aligned16(x) || !aligned4(blocks) || !aligned4(y)) return BF16X_EARG;
   if (kp_off && (!aligned4(kp_off) || !aligned4(kp_ent))) return BF16X_EARG;
+  if (bf16x_use_stream(M, out_f, in_f, true))
+    return bf16x_gemm_stream_launch((const uint16_t*)x, M, nullptr, nullptr, nullptr, nullptr, blocks, kp_off, kp_ent,
+                                    out_f, in_f, kp_off != nullptr, y_dtype == BF16X_F32, y, (hipStream_t)stream);
   if (gguf_few_rows(M, out_f, in_f)) {
     rc = bf16x_gemm_skinny2_launch((const uint16_t*)x, M, nullptr, nullptr, nullptr, nullptr, blocks, kp_off, kp_ent,
                                    out_f, in_f, kp_off != nullptr, y_dtype == BF16X_F32, y, workspace,

@@ -432,7 +432,8 @@ enum {
   BF16X_TUNE_ATTN_MFMA = 18,       /* prefill attention: 0 the scalar kernel, 1 the MFMA kernel       */
   BF16X_TUNE_CHUNK_ATOMS = 19,     /* atoms per row and chunk of the chunked few-row GEMM (8, 16, 32) */
   BF16X_TUNE_GEMM_WS_BM = 20,      /* token rows per tile of the grouped one (64, 128 or 256)             */
-  BF16X_TUNE_COUNT = 21
+  BF16X_TUNE_GEMM_STREAM_MAX = 21, /* largest M of the streaming few-row GEMM (0..16)                */
+  BF16X_TUNE_COUNT = 22
 };
 int bf16x_set_tuning(int32_t key, int64_t value);
 /* Current value of a key (-1 = automatic; also returned for an unknown key). */
