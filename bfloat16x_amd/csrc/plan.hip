@@ -10,8 +10,9 @@
 // Bound: the gathers.  An entry reads its code, sign, mantissa and emax from
 // four streams, and at one entry per ~38 elements nearly every cache line of
 // them is touched (84 MB at 14336x4096).  Measured there (1.55 M entries):
-// 15 + 4 + 18.5 us,
-// 54 us for the call with its one wait for the count; the host builder, which
+// 13 + 4 + 16 us (15
+// + 4 + 18.5 with one entry of a thread in flight at a time), 48 us for the call
+// with its one wait for the count; the host builder, which
 // copies the streams back first, takes 30-40 ms.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -27,6 +28,7 @@ using namespace bf16x;
 // iters keeps the workgroups at or below kMaxBlocks, 4 counts per thread of
 // the scan.
 constexpr int kMaxBlocks = 4096;
+constexpr int kAhead = 2;
 constexpr uint32_t kBad = 0x80000000u;     // of a workgroup's count: an entry failed its checks
 
 struct PlanGrid {
@@ -58,15 +60,35 @@ __global__ __launch_bounds__(256) void plan_count_kernel(const int32_t* __restri
   const int64_t j0 = (int64_t)blockIdx.x * 256 * iters + threadIdx.x;
   uint32_t kept = 0;
   bool bad = false;
-  for (int it = 0; it < iters; ++it) {
-    const int64_t j = j0 + 256 * (int64_t)it;
-    if (j >= n) break;
-    const int64_t p = idx[j], prev = j ? (int64_t)idx[j - 1] : -1;
-    const int v = val[j];
-    bool ok = p > prev && p >= 0 && p < N && v >= 7;
-    if (ok) ok = field(delta, p * 3, 3) == 7u && v <= (int)emax[p >> 4];
-    bad |= !ok;
-    kept += v > 7 ? 1u : 0u;
+  // kAhead entries of a thread at a time: their table words, then their
+  // gathers (the last code word's second word is only read when the field
+  // crosses into it, so all reads stay inside the stream)
+  for (int it = 0; it < iters; it += kAhead) {
+    int64_t p[kAhead], prev[kAhead];
+    int v[kAhead];
+    bool in[kAhead], ok[kAhead];
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) {
+      const int64_t j = j0 + 256 * (int64_t)(it + k);
+      in[k] = it + k < iters && j < n;
+      const int64_t jc = in[k] ? j : n - 1;
+      p[k] = idx[jc];
+      prev[k] = jc ? (int64_t)idx[jc - 1] : -1;
+      v[k] = val[jc];
+    }
+    uint32_t code[kAhead], em[kAhead];
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) {
+      ok[k] = p[k] > prev[k] && p[k] >= 0 && p[k] < N && v[k] >= 7;
+      const int64_t pc = ok[k] ? p[k] : 0;
+      code[k] = field(delta, pc * 3, 3);
+      em[k] = emax[pc >> 4];
+    }
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) {
+      bad |= in[k] && !(ok[k] && code[k] == 7u && v[k] <= (int)em[k]);
+      kept += in[k] && v[k] > 7 ? 1u : 0u;
+    }
   }
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) kept += __shfl_xor(kept, o, 64);
@@ -133,12 +155,27 @@ __global__ __launch_bounds__(256) void plan_write_kernel(
     return (int64_t)row * tpr + (c >> 16);
   };
   uint32_t base = blk_off[blockIdx.x];
+  // entry j's table words; the next iteration's are requested ahead, and an
+  // entry's gathers before the barrier that ranks it
+  const int64_t j0 = (int64_t)blockIdx.x * iters * 256 + threadIdx.x;
+  uint32_t p = 0, prev = 0;
+  int v = 0;
+  auto load = [&](int64_t j, uint32_t& pj, uint32_t& pv, int& vj) {
+    const int64_t jc = min(j, n - 1);
+    pj = (uint32_t)idx[jc];
+    pv = (uint32_t)idx[jc ? jc - 1 : 0];
+    vj = j < n ? val[jc] : 0;
+  };
+  load(j0, p, prev, v);
   for (int it = 0; it < iters; ++it) {
-    const int64_t j = ((int64_t)blockIdx.x * iters + it) * 256 + threadIdx.x;
+    const int64_t j = j0 + 256 * (int64_t)it;
     const bool in = j < n;
-    const uint32_t p = in ? (uint32_t)idx[j] : 0u;
-    const int v = in ? val[j] : 0;
     const bool keep = v > 7;
+    const uint32_t s = field(sign, p, 1), m = field(mant, (int64_t)p * 7, 7);
+    const int em = emax[p >> 4];
+    uint32_t pn, prevn;
+    int vn;
+    load(it + 1 < iters ? j + 256 : n, pn, prevn, vn);
     const uint64_t b = __ballot(keep);
     const uint32_t before = (uint32_t)__builtin_popcountll(b & ((1ull << lane) - 1ull));
     if (lane == 0) part[it & 1][wave] = (uint32_t)__builtin_popcountll(b);
@@ -152,7 +189,7 @@ __global__ __launch_bounds__(256) void plan_write_kernel(
     base += all;
     uint32_t col = 0, pcol;
     const int64_t t = in ? tile_of(p, col) : -1;
-    const int64_t t0 = in ? (j ? tile_of((uint32_t)idx[j - 1], pcol) + 1 : 0) : 0;
+    const int64_t t0 = in ? (j ? tile_of(prev, pcol) + 1 : 0) : 0;
     // a long run of empty tiles is written by the whole wave
     const int64_t gap = in ? t - t0 + 1 : 0;
     for (uint64_t m = __ballot(gap > 16); m; m &= m - 1) {
@@ -168,11 +205,12 @@ __global__ __launch_bounds__(256) void plan_write_kernel(
       for (int64_t k = tl + 1 + lane; k <= n_tiles; k += 64) tile_off[k] = (uint32_t)n_fix;
     }
     if (keep && (int64_t)o < n_fix) {
-      const uint32_t s = field(sign, p, 1), m = field(mant, (int64_t)p * 7, 7);
-      const int em = emax[p >> 4];
       sat[o] = (uint8_t)max(em - 7, 0);
       ent[o] = (col << 16) | (s << 15) | (((uint32_t)(em - v) & 0xFFu) << 7) | m;   // opqk_linear.py:375
     }
+    p = pn;
+    prev = prevn;
+    v = vn;
   }
 }
 
