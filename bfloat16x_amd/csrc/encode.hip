@@ -196,6 +196,7 @@ __global__ __launch_bounds__(256) void encode_atoms_kernel(
         *(uint16_t*)(buf + chunk_slot(lane, j >> 3) + (j & 7) * 2) = e < N ? wb[e] : (uint16_t)0;
       }
     }
+    __builtin_amdgcn_wave_barrier();                // lanes read what others wrote: kept in this order
     u32x4 q[4];
 #pragma unroll
     for (int c = 0; c < 4; ++c) q[c] = *(const u32x4*)(buf + chunk_slot(lane, c));
@@ -236,10 +237,12 @@ __global__ __launch_bounds__(256) void encode_atoms_kernel(
         emax[2 * a] = (uint8_t)t.em;
         emax[2 * a + 1] = (uint8_t)(t.em >> 8);
       }
+      __builtin_amdgcn_wave_barrier();              // the atoms are read; their place takes the words
 #pragma unroll
       for (int k = 0; k < 7; ++k) mb[lane * 7 + k] = t.m[k];
 #pragma unroll
       for (int k = 0; k < 3; ++k) mb[448 + lane * 3 + k] = t.d[k];
+      __builtin_amdgcn_wave_barrier();
       const u32x4* sc = (const u32x4*)mb;
       u32x4a* md = (u32x4a*)(mant + 7 * a0);
       md[lane] = sc[lane];
@@ -247,6 +250,7 @@ __global__ __launch_bounds__(256) void encode_atoms_kernel(
         md[64 + lane] = sc[64 + lane];
         ((u32x4a*)(delta + 3 * a0))[lane] = sc[112 + lane];
       }
+      __builtin_amdgcn_wave_barrier();              // before the next atoms overwrite them
     } else if (a < n_atoms) {
       if (a < ws) sign[a] = t.s;
       for (int k = 0; k < 7; ++k)
