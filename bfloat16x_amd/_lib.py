@@ -184,7 +184,11 @@ def ptr(t) -> int | None:
 
 
 def stream_of(device: torch.device):
-    """Raw hipStream_t of torch's current stream on `device`."""
+    """Raw hipStream_t of torch's current stream on `device`, a GPU: the
+    wrappers launch on pointers of that device's tensors, so any other device
+    is refused here."""
+    if device.type != "cuda":
+        raise ValueError(f"expected a GPU device, not {device}")
     index = device.index
     return host().stream(torch.cuda.current_device() if index is None else index)
 

@@ -6,6 +6,7 @@ import ctypes
 
 import numpy as np
 import pytest
+import torch
 
 from oracle import gguf_codec as go
 
@@ -161,3 +162,16 @@ def test_pack_ovf_bytes_match_reference(golden, case, exact):
     assert gguf.pack_ovf(x, bf16_exact=exact) == want
     if case == "dense":
         assert int(np.frombuffer(want[4:8], dtype=np.uint32)[0]) > x.shape[0] * 8   # many entries per row
+
+
+def test_host_table_is_refused_before_a_launch():
+    """A table on the host has no step-major plan: asking for one is refused
+    where the launch takes its stream, before a kernel sees host pointers."""
+    rng = np.random.default_rng(5)
+    w = (rng.standard_t(3, (32, 256)) * 0.02).astype(np.float32)
+    t = gguf.device_ovf(gguf.pack_ovf(w), gguf.quantize_blocks(w), "cpu")
+    with pytest.raises(ValueError):
+        t.kplan(256)
+    for dev in ("cpu", "meta"):
+        with pytest.raises(ValueError):
+            _lib.stream_of(torch.device(dev))
