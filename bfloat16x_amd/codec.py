@@ -244,7 +244,10 @@ def build_plan_host(packed: dict, check: int = 1, device=None) -> Bf16xPlan:
     if int(packed.get("sub", SUB)) != SUB:
         raise _lib.Bf16xError(_lib.ESUB, "build_plan_host")
     if check == 1 and _on_device(packed, device):
-        return _build_plan_on_device(packed)
+        # launches and the count's copy go to the dict's GPU, which need not be
+        # the current one: the host builder only copies, so it never had to be
+        with torch.cuda.device(packed["delta_ovf_idx"].device):
+            return _build_plan_on_device(packed)
     sign = _host_i32(packed["sign_packed"])
     mant = _host_i32(packed["mant_packed"])
     delta = _host_i32(packed["delta_packed"])

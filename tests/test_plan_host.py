@@ -1,0 +1,47 @@
+"""CPU test of how the device plan builder is reached: with the dict's GPU as
+the current device, whatever was current before."""
+import contextlib
+import ctypes
+
+import torch
+
+import bfloat16x_amd as bx
+from bfloat16x_amd import _lib, codec
+
+
+def test_device_builder_runs_on_the_dicts_gpu(monkeypatch):
+    """A dict on a GPU that is not the current one: its stream, both launches
+    and the wait for the count belong inside a guard for the dict's device.
+    (A null stream handle means the current device's default stream.)"""
+    d = bx.bf16x_quantize(torch.randn(8, 96, generator=torch.Generator().manual_seed(0)))
+    d["delta_ovf_idx"], d["delta_ovf_val"] = torch.tensor([5], dtype=torch.int32), torch.tensor([9], dtype=torch.uint8)
+    current, seen = ["another"], []
+
+    @contextlib.contextmanager
+    def guard(device):
+        before, current[0] = current[0], device
+        yield
+        current[0] = before
+
+    class Lib:
+        def __getattr__(self, name):
+            return getattr(_lib._LIB, name)
+
+        def bf16x_plan_device_count(self, *a):
+            seen.append(("count", current[0]))
+            ctypes.c_int64.from_address(a[9]).value = 0
+            return 0
+
+        def bf16x_plan_device_write(self, *a):
+            seen.append(("write", current[0]))
+            return 0
+
+    _lib.lib()
+    monkeypatch.setattr(codec, "_on_device", lambda packed, device: True)
+    monkeypatch.setattr(torch.cuda, "device", guard)
+    monkeypatch.setattr(_lib, "lib", lambda stub=Lib(): stub)
+    monkeypatch.setattr(_lib, "stream_of", lambda dev: seen.append(("stream", current[0])) or 0)
+    plan = bx.build_plan_host(d, device="cuda:1")
+    where = d["delta_ovf_idx"].device
+    assert seen == [("stream", where), ("count", where), ("write", where)]
+    assert plan.n_fix == 0 and current == ["another"]
