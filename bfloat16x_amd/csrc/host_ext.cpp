@@ -46,6 +46,14 @@ int32_t x_code(c10::ScalarType t) {
   return t == c10::kBFloat16 ? BF16X_BF16 : t == c10::kHalf ? BF16X_F16 : t == c10::kFloat ? BF16X_F32 : -1;
 }
 
+// The GIL given up for the scope (and taken again when an exception leaves it):
+// a launch or an allocation may wait for the GPU, and a host callback that the
+// GPU waits for may need Python.
+struct WithoutGil {
+  PyThreadState* state = PyEval_SaveThread();
+  ~WithoutGil() { PyEval_RestoreThread(state); }
+};
+
 void* stream_of(int dev) { return (void*)c10::hip::getCurrentHIPStream((c10::DeviceIndex)dev).stream(); }
 
 // gemv(x, sign, mant, delta, emax, tile_off, tile_ent, tile_sat, out_f, in_f,
@@ -70,20 +78,23 @@ PyObject* gemv(PyObject*, PyObject* const* a, Py_ssize_t n) {
     }
     if (out_f <= 0 || x->numel() != in_f) Py_RETURN_NONE;
     at::Tensor y;
-    if (a[11] == Py_None) {
-      y = at::empty({out_f}, tensor_of(a[1])->options().dtype(c10::kBFloat16));
-    } else {
+    if (a[11] != Py_None) {
       const at::Tensor* o = tensor_of(a[11]);
       if (!o || !on_gpu(*o, dev) || o->scalar_type() != c10::kBFloat16 || o->numel() < out_f) Py_RETURN_NONE;
       y = *o;
     }
     const at::Tensor &s = *tensor_of(a[1]), &m = *tensor_of(a[2]), &d = *tensor_of(a[3]), &e = *tensor_of(a[4]);
     auto p = [&](int i) { return exact ? plan[i]->data_ptr() : nullptr; };
-    const int rc = bf16x_gemv(x->data_ptr(), x_code(x->scalar_type()), (const int32_t*)s.data_ptr(), s.numel(),
-                              (const int32_t*)m.data_ptr(), m.numel(), (const int32_t*)d.data_ptr(), d.numel(),
-                              (const uint8_t*)e.data_ptr(), e.numel(), (const uint32_t*)p(0), (const uint32_t*)p(1),
-                              (const uint8_t*)p(2), out_f, in_f, (int32_t)sub,
-                              exact ? BF16X_EXACT : BF16X_SATURATED, (uint16_t*)y.data_ptr(), stream_of(dev));
+    int rc;
+    {
+      const WithoutGil no_gil;                  // (the caller's references keep the tensors)
+      if (!y.defined()) y = at::empty({out_f}, s.options().dtype(c10::kBFloat16));
+      rc = bf16x_gemv(x->data_ptr(), x_code(x->scalar_type()), (const int32_t*)s.data_ptr(), s.numel(),
+                      (const int32_t*)m.data_ptr(), m.numel(), (const int32_t*)d.data_ptr(), d.numel(),
+                      (const uint8_t*)e.data_ptr(), e.numel(), (const uint32_t*)p(0), (const uint32_t*)p(1),
+                      (const uint8_t*)p(2), out_f, in_f, (int32_t)sub, exact ? BF16X_EXACT : BF16X_SATURATED,
+                      (uint16_t*)y.data_ptr(), stream_of(dev));
+    }
     if (rc != 0) Py_RETURN_NONE;
     return THPVariable_Wrap(std::move(y));
   } catch (...) {
@@ -148,8 +159,11 @@ PyObject* invoke(int (*f)(A...), PyObject* const* a, Py_ssize_t n, std::index_se
     std::tuple<std::decay_t<A>...> v;
     if (!(from_py(a[I], std::get<I>(v)) && ...)) return nullptr;
     int rc;
-    Py_BEGIN_ALLOW_THREADS rc = f(std::get<I>(v)...);
-    Py_END_ALLOW_THREADS return PyLong_FromLong(rc);
+    {
+      const WithoutGil no_gil;
+      rc = f(std::get<I>(v)...);
+    }
+    return PyLong_FromLong(rc);
   } catch (const std::exception& e) {
     return PyErr_Format(PyExc_RuntimeError, "%s", e.what());
   }

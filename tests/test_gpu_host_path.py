@@ -1,5 +1,8 @@
 """The native call path of the wrappers (ordinary tensors) against their Python
 path: the same bits for every form both take, and the same refusals."""
+import sys
+import threading
+
 import pytest
 import torch
 
@@ -99,3 +102,33 @@ def test_stream_and_capture(bx, weight):  # noqa: F811
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(y, -want if k % 2 == 0 else want)
+
+
+def test_gemv_lets_other_threads_run(bx, weight):  # noqa: F811
+    """The native GEMV call gives up the GIL: with the interpreter's own
+    switching off, a thread that waits for it runs between two instructions of
+    a caller that does nothing else."""
+    w, plan = weight
+    x = torch.zeros(IN_F, dtype=torch.bfloat16, device=DEV)
+    out = torch.empty(OUT_F, dtype=torch.bfloat16, device=DEV)       # (freeing a result would give it up too)
+    args = (x, *w, plan.tile_off, plan.tile_ent, plan.tile_sat, OUT_F, IN_F, 16, out)
+    gemv = bx._lib.host().gemv
+    assert gemv(*args) is out
+    go, ran = threading.Lock(), []
+    go.acquire()
+    t = threading.Thread(target=lambda: (go.acquire(), ran.append(1)))
+    t.start()
+    interval = sys.getswitchinterval()
+    sys.setswitchinterval(1000.0)
+    try:
+        go.release()
+        for _ in range(20000):                       # (some tens suffice)
+            gemv(*args)
+            if ran:
+                break
+        met = bool(ran)
+    finally:
+        sys.setswitchinterval(interval)
+    t.join()
+    torch.cuda.synchronize()
+    assert met
