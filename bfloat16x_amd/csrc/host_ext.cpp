@@ -57,7 +57,8 @@ struct WithoutGil {
 void* stream_of(int dev) { return (void*)c10::hip::getCurrentHIPStream((c10::DeviceIndex)dev).stream(); }
 
 // gemv(x, sign, mant, delta, emax, tile_off, tile_ent, tile_sat, out_f, in_f,
-// sub, out): y, or None when the Python path has to take the call
+// sub, out): y; None when the Python path has to take the call; the status (an
+// int) when the launch was made and the runtime reports an error
 PyObject* gemv(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (n != 12) Py_RETURN_NONE;
   try {
@@ -95,7 +96,8 @@ PyObject* gemv(PyObject*, PyObject* const* a, Py_ssize_t n) {
                       (const uint8_t*)p(2), out_f, in_f, (int32_t)sub, exact ? BF16X_EXACT : BF16X_SATURATED,
                       (uint16_t*)y.data_ptr(), stream_of(dev));
     }
-    if (rc != 0) Py_RETURN_NONE;
+    if (rc < 0) Py_RETURN_NONE;                 // refused before the launch
+    if (rc > 0) return PyLong_FromLong(rc);     // a runtime error, reported after it: not to be launched again
     return THPVariable_Wrap(std::move(y));
   } catch (...) {
     Py_RETURN_NONE;

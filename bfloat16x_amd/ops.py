@@ -157,6 +157,8 @@ def bf16x_gemv(x, sign, mant, delta, emax, out_f, in_f, plan: Bf16xPlan | None =
         y = _lib.host().gemv(x, sign, mant, delta, emax, plan.tile_off, plan.tile_ent, plan.tile_sat, out_f, in_f,
                              sub, out)
     if y is not None:
+        if isinstance(y, int):
+            _lib.check(y, "bf16x_gemv")
         return y
     s, m, d, e = _streams(sign, mant, delta, emax)
     xx = _dev_tensor(x, "x", tuple(_X_DTYPES)).reshape(-1)

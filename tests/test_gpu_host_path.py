@@ -1,5 +1,6 @@
 """The native call path of the wrappers (ordinary tensors) against their Python
 path: the same bits for every form both take, and the same refusals."""
+import ctypes
 import sys
 import threading
 
@@ -132,3 +133,31 @@ def test_gemv_lets_other_threads_run(bx, weight):  # noqa: F811
     t.join()
     torch.cuda.synchronize()
     assert met
+
+
+def test_runtime_error_is_raised_and_not_launched_again(bx, weight, monkeypatch):  # noqa: F811
+    """A runtime error is reported after the kernel was enqueued: the wrapper
+    raises it and does not run the GEMV a second time.  The error is one left
+    pending in the runtime by a refused host call (no such device)."""
+    w, plan = weight
+    x = torch.zeros(IN_F, dtype=torch.bfloat16, device=DEV)
+    out = torch.empty(OUT_F, dtype=torch.bfloat16, device=DEV)
+    with open("/proc/self/maps") as f:
+        hip = ctypes.CDLL(next(ln.split()[-1] for ln in f if "libamdhip64" in ln))
+    lib, again = bx._lib.lib(), []
+
+    class Lib:
+        def __getattr__(self, name):
+            if name == "bf16x_gemv":
+                again.append(name)
+            return getattr(lib, name)
+
+    bx.bf16x_gemv(x, *w, OUT_F, IN_F, plan=plan, out=out)
+    monkeypatch.setattr(bx._lib, "lib", lambda: Lib())
+    pending = hip.hipSetDevice(1 << 12)
+    assert pending > 0
+    with pytest.raises(bx.Bf16xError) as e:
+        bx.bf16x_gemv(x, *w, OUT_F, IN_F, plan=plan, out=out)
+    assert e.value.status == pending and not again
+    torch.cuda.synchronize()
+    bx.bf16x_gemv(x, *w, OUT_F, IN_F, plan=plan, out=out)             # the error was taken with the report
