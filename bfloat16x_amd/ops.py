@@ -386,6 +386,12 @@ def _gemm_launch(x2, s, m, d, e, out_f, in_f, plan, y, y_dtype, sub=16):
     _lib.check(st, "bf16x_gemm")
 
 
+def _terms_in_one_launch(M: int, in_f: int) -> bool:
+    """Whether the 2 M rows of both terms stay inside the kernels' 32-bit
+    offsets: those of x in operand order, whose rows are padded to 32."""
+    return -(-2 * M // 32) * 32 * in_f * 2 < 0xFFFFFFFF
+
+
 def _gemm_terms(x2, s, m, d, e, out_f, in_f, plan, sub):
     """x2 (fp16 or fp32) . W^T in x2's dtype: x = hi + lo as two bf16 terms
     (exact for fp16, 16 significant bits for fp32), the products in fp32.
@@ -408,7 +414,7 @@ def _gemm_terms(x2, s, m, d, e, out_f, in_f, plan, sub):
     hi = terms.data_ptr()
     _lib.check(H.bf16x_split_terms(x2, code, M * in_f, hi, hi + 2 * M * in_f, st), "bf16x_split_terms")
     parts = torch.empty(2 * M, out_f, dtype=torch.float32, device=dev)
-    if 2 * M * in_f * 2 < 0xFFFFFFFF:
+    if _terms_in_one_launch(M, in_f):
         _gemm_launch(terms, s, m, d, e, out_f, in_f, plan, parts, _lib.F32, sub)
     else:
         for k in range(2):

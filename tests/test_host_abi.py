@@ -209,6 +209,33 @@ def test_gpu_entry_points_validate_before_launch():
     assert lf(o_out_f=4096, nh=16, of=(16 + 2 * KV) * 128) == _lib.ESHAPE
 
 
+@pytest.mark.skipif(torch.cuda.is_available(), reason="calls that are not refused reach a launch")
+@pytest.mark.parametrize("in_f", [64, 704, 4160, 65472])
+def test_terms_of_one_launch_are_never_refused(in_f):
+    """fp16 / fp32 activations: where the 2 M rows of the two terms go into one
+    launch, bf16x_gemm takes 2 M rows, and elsewhere the M rows of each.  The
+    rows around 4 GiB of terms; without a GPU an accepted call ends at its
+    launch (a positive status), before any pointer is used."""
+    lib, fake = _lib.lib(), ctypes.c_void_p(4096)
+    out_f = 64
+    n = out_f * in_f
+    w = [v for b in (1, 7, 3) for v in (fake, dc.stream_words(n, b))] + [fake, n // 16]
+
+    def refused(rows):
+        return lib.bf16x_gemm(fake, _lib.BF16, rows, *w, None, None, out_f, in_f, 16, _lib.SATURATED, fake,
+                              _lib.F32, fake, 1 << 60, None) < 0
+    top = 0xFFFFFFFF // (2 * in_f)                                   # rows of 4 GiB
+    assert not refused(top // 64 * 32) and refused(top + 1)
+    one = 0
+    for rows in range((top - 40) // 2 * 2, top + 41, 2):
+        if bx.ops._terms_in_one_launch(rows // 2, in_f):
+            one = rows
+            assert not refused(rows), rows
+        else:
+            assert not refused(rows // 2), rows
+    assert one >= top - 33
+
+
 def test_wrappers_refuse_cpu_tensors():
     d = bx.bf16x_quantize(torch.randn(8, 64))
     with pytest.raises(ValueError):
