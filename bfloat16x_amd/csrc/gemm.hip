@@ -615,7 +615,7 @@ extern "C" int bf16x_gguf_kplan_build(const uint32_t* row_off, const uint32_t* e
 }
 
 // wave-specialised kernel (gemm_ws.hip): M >= ws_rows()
-int64_t bf16x_gemm_ws_workspace(int64_t M, int64_t out_f, int64_t in_f, bool terms);
+int64_t bf16x_gemm_ws_workspace(int64_t M, int64_t out_f, int64_t in_f, bool terms, bool gg);
 int bf16x_gemm_ws_launch(const void* x, int32_t x_dtype, int64_t M, const uint32_t* s, const uint32_t* m,
                          const uint32_t* d, const uint16_t* e, const uint8_t* blocks, const uint32_t* kp_off,
                          const uint32_t* kp_ent, int64_t out_f, int64_t in_f, bool exact, bool yf32, void* y,
@@ -728,7 +728,7 @@ extern "C" int64_t bf16x_gemm_workspace(int64_t M, int64_t out_f, int64_t in_f) 
   if (bf16x_use_stream(M, out_f, in_f, false)) return 0;
   if (use_skinny2(M, out_f, in_f)) return bf16x_gemm_skinny2_workspace(M, out_f, in_f, false);
   if (M <= skinny_rows()) return 0;
-  if (use_ws(M, out_f, in_f)) return bf16x_gemm_ws_workspace(M, out_f, in_f, false);
+  if (use_ws(M, out_f, in_f)) return bf16x_gemm_ws_workspace(M, out_f, in_f, false, false);
   const GemmShape g = gemm_shape(M, out_f, in_f);
   return g.nsplit > 1 ? (int64_t)g.nsplit * M * out_f * 4 : 0;
 }
@@ -832,7 +832,7 @@ extern "C" int64_t bf16x_gemm_terms_workspace(int64_t M, int64_t out_f, int64_t 
   if (!ws_groups(in_f) || !use_ws(2 * M, out_f, in_f) || tiles_per_row(in_f) != 1) return BF16X_ESHAPE;
   // 32-bit buffer offsets, as in bf16x_gemm
   if (out_f * (in_f >> 5) * 28 >= (int64_t)0xFFFFFFFF || 2 * M * in_f * 2 >= (int64_t)0xFFFFFFFF) return BF16X_ESHAPE;
-  return bf16x_gemm_ws_workspace(M, out_f, in_f, true);
+  return bf16x_gemm_ws_workspace(M, out_f, in_f, true, false);
 }
 
 extern "C" int bf16x_gemm_terms(const void* x, int32_t x_dtype, int64_t M, const int32_t* sign, int64_t n_sign,

@@ -581,9 +581,9 @@ void gemm_ws4_kernel(
     // group, taken as one list of their concatenated entries: entry t belongs
     // to step u(t) = (t >= c[0]) + (t >= c[1]) + (t >= c[2]).  Lane l loads
     // entries l, l + 64, .. ahead: NE of them in any case (one entry in 32
-    // elements, more than a dict's 1 in 38 to 108), and up to NP where the list
+    // elements, more than a dict's 1 in 43 to 108), and up to NP where the list
     // goes on, a uniform branch each.  A GGUF table has every element seven
-    // steps down in it, 1 in 27 to 54, and most of its lists are longer: with
+    // steps down in it, 1 in 22 to 54, and most of its lists are longer: with
     // the rest of them loaded where they are written, each such load draining
     // the atoms in flight, 14336x4096 lossless took 83.4 us at M = 300 (74.1
     // here) and 39.0 at M = 64 (36.0).
@@ -1002,19 +1002,34 @@ int64_t ws_resident() {
 
 // Token rows per tile of the grouped kernel.  A tile of 64 tokens decodes its W
 // rows in about the time of a 128-token tile (the decode sets the pace), a
-// 256-token tile in a third more, so a tile covers all tokens up to 256 unless
-// two smaller token tiles still leave every CU at most one block before K is
-// split (C / 4: their shorter K ranges and smaller partials then win).
+// 256-token tile in a third more, so a tile covers all tokens up to 256.  Two
+// smaller token tiles decode every W row twice and win only where that is a
+// short part of the launch: where they still leave every CU at most one block
+// before K is split (C / 4: shorter K ranges and smaller partials), and a
+// block's K range is short: at most 12 column groups for a dict; for GGUF
+// blocks, whose decode (46-byte blocks, twice the plan entries) takes longer,
+// 4 with 64-token and 6 with 128-token tiles.
 // Measured, exact, 64 / 128 / 256-token tiles (us): 14336x4096 M = 64 38.6 /
 // 42.1 / 48.7, M = 128 52.8 / 45.3 / 51.1, M = 191 74.9 / 60.7 / 54.3;
-// 4096x4096 (32 row tiles) M = 64 22.6 / 24.1 / 28.8, M = 128 23.8 / 24.9 /
-// 29.5, M = 191 30.1 / 27.3 / 30.7.
-int64_t ws_tile_rows(int64_t M, int64_t nt, int64_t C, bool terms) {
+// 4096x4096 (32 row tiles, two smaller tiles: 4 groups) M = 64 22.6 / 24.1 /
+// 28.8, M = 128 23.8 / 24.9 / 29.5, M = 191 30.1 / 27.3 / 30.7.  Time of two
+// 64-token tiles over one of 128 at M = 101, and of two of 128 over one of 256
+// at M = 160, by groups: dict exact 5 0.97 / 0.89, 8 0.99 / 0.92, 12 1.05 /
+// 1.02, 14 1.05 / 1.05 (saturated 0.90 / 0.86, 0.94 / 0.89, 0.94 / 1.00, 1.08
+// / 1.01); GGUF lossless 4 0.99 / 0.98, 5 1.06 / 0.97, 6 1.09 / 1.03, 8 1.12 /
+// 1.03, 14 1.27 / 1.16 (4096x14336: M = 101 48.4 against 38.3, M = 160 56.5
+// against 48.4); without a table 5 1.01 / 0.96, 6 1.03 / 0.98, 8 1.00 / 1.01, 14
+// 1.12 / 1.13.
+constexpr int64_t kMaxSplit = 16;
+int64_t ws_tile_rows(int64_t M, int64_t nt, int64_t units, int64_t C, bool terms, bool gg) {
   const int64_t t = tuning(BF16X_TUNE_GEMM_WS_BM);
   if (t == 64 || t == 128 || (t == 256 && !terms)) return t;
   for (int64_t bm = 64; bm < 256; bm *= 2) {
     const int64_t mt = (M + bm - 1) / bm;
-    if (mt == 1 || (mt == 2 && mt * nt <= C / 4)) return bm;
+    if (mt == 1) return bm;
+    if (mt > 2 || mt * nt > C / 4) continue;
+    const int64_t s = std::min<int64_t>(C / (mt * nt), kMaxSplit);      // (as ws_shape splits K)
+    if ((units + s - 1) / s <= (!gg ? 12 : bm == 64 ? 4 : 6)) return bm;
   }
   return terms ? 128 : 256;    // two terms: the operands of a 256-token tile do not fit the registers
 }
@@ -1028,18 +1043,17 @@ int64_t ws_tile_rows(int64_t M, int64_t nt, int64_t C, bool terms) {
 // only for those 128 tiles.  BF16X_TUNE_GEMM_WS_SPLIT > 0 splits every tile
 // into that many K ranges instead; BF16X_TUNE_GEMM_WS_RESIDENT > 0 replaces
 // the resident block count (tests reach the mixed plan with few tiles).
-WsShape ws_shape(int64_t M, int64_t out_f, int64_t in_f, bool terms = false) {
+WsShape ws_shape(int64_t M, int64_t out_f, int64_t in_f, bool terms, bool gg) {
   WsShape w;
   w.grouped = ws_grouped(in_f);
   const int64_t forced_c = tuning(BF16X_TUNE_GEMM_WS_RESIDENT);
   // (the reduction indexes the split tiles' elements in 32 bits)
   const int64_t C = forced_c > 0 ? std::min<int64_t>(forced_c, 32768) : ws_resident();
   const int64_t nt = (out_f + kBN - 1) / kBN;
-  const int64_t bm = w.grouped ? ws_tile_rows(M, nt, C, terms) : kBM;
-  const int64_t mt = (M + bm - 1) / bm;
-  const int64_t S = in_f / kStep, tiles = mt * nt;
-  const int64_t units = w.grouped ? S / kGroup : S;
-  const int64_t max_split = std::max<int64_t>(1, std::min<int64_t>(16, w.grouped ? units : units / 4));
+  const int64_t S = in_f / kStep, units = w.grouped ? S / kGroup : S;
+  const int64_t bm = w.grouped ? ws_tile_rows(M, nt, units, C, terms, gg) : kBM;
+  const int64_t mt = (M + bm - 1) / bm, tiles = mt * nt;
+  const int64_t max_split = std::max<int64_t>(1, std::min<int64_t>(kMaxSplit, w.grouped ? units : units / 4));
   int64_t f = tiles % C, s = f ? std::min<int64_t>(C / f, max_split) : 1;
   const int64_t forced = tuning(BF16X_TUNE_GEMM_WS_SPLIT);
   if (forced > 0 && tiles <= 32768) {
@@ -1070,8 +1084,8 @@ int64_t ws_xop_bytes(int64_t M, int64_t in_f) { return ((M + 31) / 32) * 32 * in
 }  // namespace
 
 // terms: x is fp16 or fp32, multiplied as two bf16 terms (grouped kernel only)
-int64_t bf16x_gemm_ws_workspace(int64_t M, int64_t out_f, int64_t in_f, bool terms) {
-  const WsShape w = ws_shape(M, out_f, in_f, terms);
+int64_t bf16x_gemm_ws_workspace(int64_t M, int64_t out_f, int64_t in_f, bool terms, bool gg) {
+  const WsShape w = ws_shape(M, out_f, in_f, terms, gg);
   return ws_xop_bytes(M, in_f) * (terms ? 2 : 1) +
          (w.nsplit > 1 ? (int64_t)w.nsplit * w.g.ltiles * ((int64_t)w.g.bm * kBN) * 4 : 0);
 }
@@ -1085,10 +1099,11 @@ int bf16x_gemm_ws_launch(const void* x, int32_t x_dtype, int64_t M, const uint32
                          const uint32_t* kp_ent, int64_t out_f, int64_t in_f, bool exact, bool yf32, void* y,
                          void* workspace, int64_t workspace_bytes, hipStream_t st) {
   const bool terms = x_dtype != BF16X_BF16;
-  const WsShape w = ws_shape(M, out_f, in_f, terms);
+  const WsShape w = ws_shape(M, out_f, in_f, terms, blocks != nullptr);
   if (terms && (!w.grouped || blocks)) return BF16X_ESHAPE;
   const int64_t xop = ws_xop_bytes(M, in_f);
-  if (!workspace || !aligned16(workspace) || workspace_bytes < bf16x_gemm_ws_workspace(M, out_f, in_f, terms))
+  if (!workspace || !aligned16(workspace) ||
+      workspace_bytes < bf16x_gemm_ws_workspace(M, out_f, in_f, terms, blocks != nullptr))
     return BF16X_ECAPACITY;
   if (xop >= (int64_t)0xFFFFFFFF) return BF16X_ESHAPE;
   if (w.grid > INT32_MAX) return BF16X_ESHAPE;

@@ -629,7 +629,7 @@ extern "C" int bf16x_gguf_gemv_lossless(const void* x, int32_t x_dtype, const ui
 // (46-byte blocks, zero-marker decode).
 // The lossless table enters as the step-major plan of bf16x_gguf_kplan_build.
 // ---------------------------------------------------------------------------
-int64_t bf16x_gemm_ws_workspace(int64_t M, int64_t out_f, int64_t in_f, bool terms);
+int64_t bf16x_gemm_ws_workspace(int64_t M, int64_t out_f, int64_t in_f, bool terms, bool gg);
 int bf16x_gemm_ws_launch(const void* x, int32_t x_dtype, int64_t M, const uint32_t* s, const uint32_t* m,
                          const uint32_t* d, const uint16_t* e, const uint8_t* blocks, const uint32_t* kp_off,
                          const uint32_t* kp_ent, int64_t out_f, int64_t in_f, bool exact, bool yf32, void* y,
@@ -669,7 +669,7 @@ extern "C" int64_t bf16x_gguf_gemm_workspace(int64_t M, int64_t out_f, int64_t i
   if (M <= 0 || out_f <= 0 || in_f < 64 || (in_f % 64) != 0) return 0;
   if (bf16x_use_stream(M, out_f, in_f, true)) return 0;
   if (gguf_few_rows(M, out_f, in_f)) return bf16x_gemm_skinny2_workspace(M, out_f, in_f, true);
-  return bf16x_gemm_ws_workspace(M, out_f, in_f, false);
+  return bf16x_gemm_ws_workspace(M, out_f, in_f, false, true);
 }
 
 extern "C" int bf16x_gguf_gemm(const void* x, int32_t x_dtype, int64_t M, const uint8_t* blocks, int64_t n_bytes,

@@ -236,6 +236,29 @@ def test_terms_of_one_launch_are_never_refused(in_f):
     assert one >= top - 33
 
 
+# (rows, in_f of 4096 output rows) and the tokens per tile: two small tiles while
+# a block's K range is short (in_f / 1024 column groups each), one tile that
+# covers all rows beyond; the line of GGUF blocks lies lower
+@pytest.mark.parametrize("M,in_f,dict_rows,gguf_rows", [
+    (101, 4096, 64, 64), (101, 5120, 64, 128), (101, 12288, 64, 128), (101, 12544, 128, 128),
+    (160, 6144, 128, 128), (160, 6400, 128, 256), (160, 12288, 128, 256), (160, 14336, 256, 256), (65, 256, 64, 64),
+    (300, 4096, 256, 256)])
+def test_tile_rows_of_the_grouped_gemm(tune, M, in_f, dict_rows, gguf_rows):
+    """Read from the workspace: x in operand order, and the fp32 partials of
+    every split tile."""
+    tune(gemm_ws_resident=256)
+    lib = _lib.lib()
+
+    def want(bm):
+        tiles = -(-M // bm) * 32
+        split = min(256 // tiles, 16, in_f // 256)
+        units = in_f // 256
+        used = -(-units // -(-units // split))                        # ranges that hold a group
+        return -(-M // 32) * 32 * in_f * 2 + (used * tiles * bm * 128 * 4 if used > 1 else 0)
+    assert lib.bf16x_gemm_workspace(M, 4096, in_f) == want(dict_rows)
+    assert lib.bf16x_gguf_gemm_workspace(M, 4096, in_f) == want(gguf_rows)
+
+
 def test_wrappers_refuse_cpu_tensors():
     d = bx.bf16x_quantize(torch.randn(8, 64))
     with pytest.raises(ValueError):
