@@ -35,7 +35,7 @@ def _bf16_bits_host(w: torch.Tensor) -> torch.Tensor:
 
 
 def _quantize_device(w: torch.Tensor) -> dict:
-    """The device encoder (bf16x_encode): outputs on w's GPU."""
+    """The device encoder (bf16x_encode_streams, bf16x_encode_table): outputs on w's GPU."""
     out_f, in_f = (int(s) for s in w.shape)
     n = out_f * in_f
     dev = w.device

@@ -1,4 +1,5 @@
-"""GPU tests of the device encoder (bf16x_encode): the dict of a GPU weight
+"""GPU tests of the device encoder (bf16x_encode_streams, bf16x_encode_table and
+both in one, bf16x_encode): the dict of a GPU weight
 is byte-identical to the reference's golden dicts and to the host encoder,
 for odd sizes (N not a multiple of 32, N < 32), special values (+-0,
 denormals, inf, NaN, exponent 255), configuration 1 and the headline shape."""
@@ -103,3 +104,39 @@ def test_device_encoder_segments(bx, shape, kind):
     d = bx.bf16x_quantize(w.to(DEV))
     same_dict(d, bx.bf16x_quantize(w), (kind, shape))
     assert (d["delta_ovf_idx"].numel() == 0) == (kind == "flat")
+
+
+@pytest.mark.parametrize("kind", ["bench", "spread", "flat"])
+def test_combined_entry_and_its_capacity(bx, kind):
+    """bf16x_encode: the streams and the table in one call; with room for fewer
+    entries than there are it writes those that fit and the whole count, and a
+    second call with that count has them all."""
+    shape = (65, 1056)
+    bits = {"bench": lambda: dc.bench_weight_bits(*shape, seed=7), "spread": lambda: spread_bits(shape, 8),
+            "flat": lambda: np.full(shape, 0x3C00, np.uint16)}[kind]()
+    w = torch.from_numpy(bits.view(np.int16).copy()).view(torch.bfloat16)
+    want, L, n = bx.bf16x_quantize(w), bx._lib.lib(), bits.size
+    k = want["delta_ovf_idx"].numel()
+    wd = w.to(DEV)
+    ws = torch.empty(int(L.bf16x_encode_workspace(*shape)) // 4 + 4, dtype=torch.int32, device=DEV)
+
+    def encode(cap):
+        d = {f: torch.full((bx.stream_words(n, b),), -1, dtype=torch.int32, device=DEV)
+             for f, b in (("sign_packed", 1), ("mant_packed", 7), ("delta_packed", 3))}
+        d["emax"] = torch.full((-(-n // 16),), 255, dtype=torch.uint8, device=DEV)
+        idx = torch.full((k + 8,), -1, dtype=torch.int32, device=DEV)
+        val = torch.zeros(k + 8, dtype=torch.uint8, device=DEV)
+        count = torch.full((1,), -1, dtype=torch.int64, device=DEV)
+        st = L.bf16x_encode(wd.data_ptr(), *shape, 16, *(v for f in ("sign_packed", "mant_packed", "delta_packed", "emax")
+                                                         for v in (d[f].data_ptr(), d[f].numel())),
+                            idx.data_ptr() if cap else None, val.data_ptr() if cap else None, cap, count.data_ptr(),
+                            ws.data_ptr(), ws.numel() * 4, bx._lib.stream_of(wd.device))
+        assert st == 0 and int(count) == k
+        for f in ("sign_packed", "mant_packed", "delta_packed", "emax"):
+            assert torch.equal(d[f].cpu(), want[f]), f
+        m = min(cap, k)
+        assert torch.equal(idx[:m].cpu(), want["delta_ovf_idx"][:m]) and torch.equal(val[:m].cpu(),
+                                                                                     want["delta_ovf_val"][:m])
+        assert bool((idx[m:] == -1).all()) and bool((val[m:] == 0).all())      # nothing past the capacity
+    for cap in (0, 1, k // 2, max(k - 1, 0), k, k + 3):
+        encode(cap)

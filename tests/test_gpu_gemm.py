@@ -22,8 +22,10 @@ def _np(d):
     return {k: (v.numpy() if isinstance(v, torch.Tensor) else v) for k, v in d.items()}
 
 
-# (M, out_f, in_f): every tile configuration (M <= 32, <= 64, <= 128, > 128),
-# ragged M and out_f, the C3 prefill shapes at reduced out_f
+# (M, out_f, in_f): the dispatch's kernels from one row to 2048 (few-row, grouped
+# wave-specialised with its token tiles, one step at a time at 300 x 640),
+# ragged M and out_f, the C3 prefill shapes at reduced out_f; the tiled kernel
+# has its tests in test_gpu_gemm_tiled.py
 CASES = [(1, 128, 64), (5, 96, 128), (16, 512, 4096), (33, 200, 1536), (64, 1024, 4096), (100, 300, 1536),
          (128, 256, 14336), (256, 1024, 4096), (300, 130, 640), (512, 512, 4096), (2048, 256, 4096)]
 
@@ -51,8 +53,9 @@ def test_gemm_saturated_and_exact(bx, M, out_f, in_f, path):
 
 
 def test_gemm_exact_dense_overflow(bx):
-    """A weight with many overflow entries per row (every atom has several),
-    so the plan window refills inside one atom."""
+    """A weight with many overflow entries per row (every atom has several):
+    runs longer than the few-row kernel's preload (48 rows) and than the
+    grouped kernel's lists (256 rows)."""
     out_f, in_f, M = 64, 1024, 48
     rng = np.random.default_rng(7)
     bits = dc.bench_weight_bits(out_f, in_f, seed=7)
@@ -143,8 +146,9 @@ def test_gemm_full_size(bx):
 
 @pytest.mark.parametrize("M", [32, 64, 100])
 def test_gemm_few_rows_identity_is_bit_exact(bx, M):
-    """The few-row kernel (M <= 128): x = rows of I select W columns, so the
-    decode that feeds its MFMA is checked bit for bit, exact and saturated."""
+    """The chunked, 16x16x32 and grouped kernels the dispatch takes at these
+    rows: x = rows of I select W columns, so the decode that feeds the MFMA is
+    checked bit for bit, exact and saturated."""
     out_f, in_f = 96, 1024
     bits = with_specials(dc.bench_weight_bits(out_f, in_f, seed=M), seed=M)
     bits[(bits & 0x7F00) == 0x7F00] = 0x3F80
@@ -165,7 +169,7 @@ def test_gemm_few_rows_identity_is_bit_exact(bx, M):
             assert np.array_equal(got, ref[:, start:start + cols]), (start, p is None)
 
 
-# The wave-specialised kernel (M >= 192): four-step groups when in_f % 256 == 0
+# The wave-specialised kernel at 192 rows and more: four-step groups when in_f % 256 == 0
 # (grouped = 1, the default there) and one-step tiles otherwise or when forced
 # (grouped = 0); K splits forced to 1 and 3 (3 leaves a shorter last split).
 @pytest.mark.parametrize("grouped", [1, 0])

@@ -2,18 +2,20 @@
 16x16x32-MFMA kernel behind bf16x_gemm, bf16x_gemm_fused.py:97 contract)
 against the oracle, through the C ABI.
 
+The tests with the `pinned` fixture run this kernel whatever the dispatch
+would take for their shapes (bf16x_gemm of the C ABI under the tuning keys).
 Beside the bf16-output checks of test_gpu_gemm.py (which also reach this
-kernel), the product is read in fp32 (fp32 activations that are exactly
-bf16 give y = the fp32 accumulation of one pass) and held to 1e-3 of the
-float64 product: a dropped or misplaced term (about 1/sqrt(in_f) of an
-output) fails it.  Rows of I pick W columns bit for bit, which pins the
-MFMA operand and result layouts and every overflow patch."""
+kernel), the product is read in fp32 and held to 1e-3 of the float64 product:
+a dropped or misplaced term (about 1/sqrt(in_f) of an output) fails it.  Rows
+of I pick W columns bit for bit, which pins the MFMA operand and result
+layouts and every overflow patch."""
 
 import numpy as np
 import pytest
 import torch
 
 from oracle import dict_codec as dc
+from tests.gemm_abi import columns_bit_for_bit, product
 from tests.test_gpu_dict import DEV, bits_tensor, check_tol, to_dev, with_specials
 
 pytestmark = pytest.mark.gpu
@@ -28,11 +30,18 @@ def bx():
 
 @pytest.fixture(autouse=True)
 def _no_row_kernel(bx, monkeypatch):
-    """bf16x_gemm runs the row-streaming kernel for M <= 16 at in_f 2048 /
-    4096 (test_gpu_gemm_rows.py) and the GEMV for one bf16 row; these tests
-    pin the 16x16x32 kernel."""
+    """ops.bf16x_gemm runs the row-streaming kernel for M <= 16 at in_f 2048 /
+    4096 (test_gpu_gemm_rows.py) and the GEMV for one bf16 row: not here."""
     monkeypatch.setattr(bx.ops, "GEMM_ROWS_MAX", 0)
     monkeypatch.setattr(bx.ops, "GEMM_ONE_ROW_GEMV", False)
+
+
+@pytest.fixture
+def pinned(tune):
+    """Up to 64 rows at in_f % 128 == 0 on the 16x16x32 kernel (an explicit
+    gemm_skinny2_max also keeps the grouped kernel off few rows of large
+    weights)."""
+    tune(gemm_skinny2_max=64, gemm_stream_max=0)
 
 
 def _np(d):
@@ -60,74 +69,69 @@ CASES = [(1, 64, 128), (2, 200, 1024), (5, 130, 4096), (16, 512, 1536), (17, 96,
 
 
 @pytest.mark.parametrize("M,out_f,in_f", CASES)
-def test_skinny2_fp32_product(bx, M, out_f, in_f):
+def test_skinny2_fp32_product(bx, pinned, M, out_f, in_f):
     print("skinny2 fp32", M, out_f, in_f, flush=True)
     bits, d, g, plan = _weight(bx, out_f, in_f, seed=M + out_f)
-    x = torch.randn(M, in_f, generator=torch.Generator().manual_seed(M)).to(torch.bfloat16).float()
+    x = torch.randn(M, in_f, generator=torch.Generator().manual_seed(M)).to(torch.bfloat16)
     dn = _np(d)
     for p, sat in ((plan, False), (None, True)):
-        y = _gemm(bx, x.to(DEV), g, out_f, in_f, p)
-        assert y.dtype == torch.float32 and y.shape == (M, out_f)
+        y = product(bx, x.to(DEV), g, out_f, in_f, p, torch.float32)
         mx, med = dc.rel_err(y.cpu().numpy(), dc.gemm_ref(dn, x.double().numpy(), saturated=sat))
         assert mx <= 1e-3 and med <= 1e-6, (sat, mx, med)
 
 
 @pytest.mark.parametrize("kq", ["1", "2"])
-@pytest.mark.parametrize("M,out_f,in_f", [(5, 130, 4096), (33, 72, 1024), (48, 384, 14336), (64, 200, 2048)])
-def test_skinny2_waves_per_row_group(bx, tune, kq, M, out_f, in_f):
+@pytest.mark.parametrize("M,out_f,in_f", [(5, 130, 4096), (20, 200, 2048), (33, 72, 1024), (48, 384, 14336),
+                                          (64, 200, 2048)])
+def test_skinny2_waves_per_row_group(bx, pinned, tune, kq, M, out_f, in_f):
     """The other wave-per-row-group counts (override skinny2_kq = 1: one wave
     walks every step of its rows; 2: two waves take alternate steps) give the
     same fp32 product: the default is 4 up to 32 rows and 2 above."""
     tune(skinny2_kq=int(kq))
     bits, d, g, plan = _weight(bx, out_f, in_f, seed=M + out_f + 7)
-    x = torch.randn(M, in_f, generator=torch.Generator().manual_seed(M + 1)).to(torch.bfloat16).float()
+    x = torch.randn(M, in_f, generator=torch.Generator().manual_seed(M + 1)).to(torch.bfloat16)
     dn = _np(d)
     for p, sat in ((plan, False), (None, True)):
-        y = _gemm(bx, x.to(DEV), g, out_f, in_f, p)
+        y = product(bx, x.to(DEV), g, out_f, in_f, p, torch.float32)
         mx, med = dc.rel_err(y.cpu().numpy(), dc.gemm_ref(dn, x.double().numpy(), saturated=sat))
         assert mx <= 1e-3 and med <= 1e-6, (kq, sat, mx, med)
 
 
-@pytest.mark.parametrize("M", [1, 16, 40, 64])
-def test_skinny2_identity_is_bit_exact(bx, M):
-    out_f, in_f = 136, 512
-    bits, d, g, plan = _weight(bx, out_f, in_f, seed=M)
-    bits = bits.copy()
-    sat = dc.decode_saturated(_np(d))
-    # the MFMA flushes subnormal inputs: compare those as zero
-    for a in (bits, sat):
-        a[(a & 0x7F80) == 0] = 0
-    for start in range(0, in_f, M):
-        cols = min(M, in_f - start)
-        eye = torch.zeros(M, in_f, dtype=torch.bfloat16)
-        eye[torch.arange(cols), start + torch.arange(cols)] = 1
-        for p, ref in ((plan, bits), (None, sat)):
-            y = _gemm(bx, eye.to(DEV), g, out_f, in_f, p)
-            got = y.contiguous().view(torch.int16).cpu().numpy().view(np.uint16)[:cols].T.copy()
-            got[(got & 0x7F80) == 0] = 0
-            assert np.array_equal(got, ref[:, start:start + cols]), (start, p is None)
+# one, two and four token blocks; the default waves per row group and both others
+@pytest.mark.parametrize("kq", [-1, 1, 2])
+@pytest.mark.parametrize("M", [1, 16, 17, 32, 40, 64])
+def test_skinny2_identity_is_bit_exact(bx, pinned, tune, M, kq):
+    tune(skinny2_kq=kq)
+    bits, d, g, plan = _weight(bx, 136, 512, seed=M)
+    columns_bit_for_bit(bx, g, bits, plan, M)
+    columns_bit_for_bit(bx, g, dc.decode_saturated(_np(d)).reshape(136, 512), None, M)
 
 
 def test_skinny2_matches_previous_kernel(bx):
-    """Same inputs through the 32x32-MFMA few-row kernel (selected by the
-    override gemm_skinny2_max = 0): both accumulate in fp32, so the bf16
-    outputs agree to within one rounding of either."""
+    """Same inputs through the chunked kernel that the dispatch takes and, in
+    its place, the 16x16x32 and the 32x32-MFMA few-row kernels (overrides): all
+    accumulate in fp32, so the bf16 outputs agree to within one rounding."""
     out_f, in_f, M = 320, 4096, 24
     bits, d, g, plan = _weight(bx, out_f, in_f, seed=4)
     x = torch.randn(M, in_f, generator=torch.Generator().manual_seed(4)).to(torch.bfloat16).to(DEV)
-    y2 = _gemm(bx, x, g, out_f, in_f, plan).float().cpu().numpy()
-    with bx.tuning(gemm_skinny2_max=0):
-        y1 = _gemm(bx, x, g, out_f, in_f, plan).float().cpu().numpy()
+    y0 = _gemm(bx, x, g, out_f, in_f, plan).float().cpu().numpy()
+    with bx.tuning(gemm_skinny2_max=64, gemm_stream_max=0):
+        y2 = product(bx, x, g, out_f, in_f, plan).float().cpu().numpy()
+    with bx.tuning(gemm_skinny2_max=0, gemm_stream_max=0):
+        y1 = product(bx, x, g, out_f, in_f, plan).float().cpu().numpy()
     ref = dc.gemm_ref(_np(d), x.float().cpu().numpy(), saturated=False)
-    check_tol(y2, ref)
-    check_tol(y1, ref)
     ulp = np.abs(y1).astype(np.float64) * 2.0 ** -7 + 1e-6
-    assert np.all(np.abs(y1.astype(np.float64) - y2) <= ulp + 1e-3 * np.sqrt(np.mean(ref * ref)))
+    for y in (y0, y1, y2):
+        check_tol(y, ref)
+        assert np.all(np.abs(y1.astype(np.float64) - y) <= ulp + 1e-3 * np.sqrt(np.mean(ref * ref)))
 
 
-def test_skinny2_dense_overflow(bx):
+@pytest.mark.parametrize("kq", [-1, 1, 2])
+@pytest.mark.parametrize("M", [16, 20, 64])
+def test_skinny2_dense_overflow(bx, pinned, tune, M, kq):
     """Runs longer than the 128 entries a lane pair preloads: the dense loop."""
-    out_f, in_f, M = 96, 1024, 20
+    tune(skinny2_kq=kq)
+    out_f, in_f = 96, 1024
     rng = np.random.default_rng(9)
     bits = dc.bench_weight_bits(out_f, in_f, seed=9)
     tiny = rng.random(bits.shape) < 0.35
@@ -135,18 +139,7 @@ def test_skinny2_dense_overflow(bx):
     d = bx.bf16x_quantize(bits_tensor(bits))
     plan = bx.build_plan_host(d, device=DEV)
     assert plan.n_fix > out_f * in_f // 32 * 4
-    g = to_dev(d)
-    eye = torch.zeros(M, in_f, dtype=torch.bfloat16)
-    for start in range(0, in_f, M):
-        cols = min(M, in_f - start)
-        eye.zero_()
-        eye[torch.arange(cols), start + torch.arange(cols)] = 1
-        y = _gemm(bx, eye.to(DEV), g, out_f, in_f, plan)
-        got = y.contiguous().view(torch.int16).cpu().numpy().view(np.uint16)[:cols].T.copy()
-        ref = bits[:, start:start + cols].copy()
-        for a in (got, ref):
-            a[(a & 0x7F80) == 0] = 0
-        assert np.array_equal(got, ref), start
+    columns_bit_for_bit(bx, to_dev(d), bits, plan, M)
 
 
 @pytest.mark.parametrize("out_f,in_f", [(14336, 4096), (4096, 14336)])

@@ -6,18 +6,10 @@ import torch
 
 from oracle import dict_codec as dc
 from oracle import gguf_codec as go
+from tests.gemm_abi import check_product as check
 from tests.test_gpu_dict import DEV, bits_tensor, bx  # noqa: F401
 
 pytestmark = pytest.mark.gpu
-
-
-def check(y, x, w):
-    """Elementwise: one rounding to y's type (bf16: at most 2^-8 of the value)
-    and the fp32 sums' own error, 4 x 2^-24 sqrt(K) of the products' magnitude."""
-    x, w = x.double(), w.double().t().contiguous()
-    ref, mag = x @ w, x.abs() @ w.abs()
-    tol = 4 * 2.0 ** -24 * w.shape[0] ** 0.5 * mag + (2.0 ** -8 * ref.abs() if y.dtype == torch.bfloat16 else 0)
-    assert bool(((y.double() - ref).abs() <= tol).all())
 
 
 def spread(out_f, in_f, seed):

@@ -42,8 +42,9 @@ def test_split_and_add_terms(bx, dt, n, off):  # noqa: F811
 
 
 # 2 M rows on each kernel of the dispatch: 2 (one row), 16 / 18, 64; from 33
-# rows the kernel that takes both terms (tiles of 64 and 128 tokens, whole K
-# and split), except at in_f % 256 != 0; a row-offset view (contiguous, its
+# rows, or 17 where the weight has 2^25 elements, the kernel that takes both
+# terms (tiles of 64 and 128 tokens, whole K and split), except at in_f % 256
+# != 0; a row-offset view (contiguous, its
 # start aligned to one element only), which a 2-byte type splits first
 @pytest.mark.parametrize("dt", [torch.float16, torch.float32])
 @pytest.mark.parametrize("exact", [True, False])
@@ -51,7 +52,8 @@ def test_split_and_add_terms(bx, dt, n, off):  # noqa: F811
     (1, 520, 2048, -1, 1), (8, 520, 2048, -1, 0), (9, 520, 2048, -1, 1), (32, 520, 2048, -1, 0),
     (33, 520, 2048, -1, 0), (33, 520, 2048, -1, 1), (64, 130, 1024, 1, 0), (65, 300, 1024, 3, 2),
     (128, 128, 256, -1, 0), (129, 200, 768, -1, 0), (200, 520, 2048, -1, 0), (300, 96, 4096, 2, 0),
-    (100, 520, 2112, -1, 0)])
+    (100, 520, 2112, -1, 0), (16, 2048, 16384, -1, 0), (17, 2048, 16384, -1, 0), (17, 2048, 16384, -1, 1),
+    (32, 2048, 16384, -1, 0)])
 def test_gemm_terms(bx, tune, dt, exact, M, out_f, in_f, split, off):  # noqa: F811
     tune(gemm_ws_split=split)
     w = bits_tensor(dc.bench_weight_bits(out_f, in_f, seed=M))

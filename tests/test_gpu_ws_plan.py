@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 import torch
 
+from tests.gemm_abi import product
 from tests.test_gpu_dict import DEV, bits_tensor, bx, gpu_bits  # noqa: F401
 
 pytestmark = pytest.mark.gpu
@@ -43,21 +44,8 @@ def test_entries_bit_for_bit(bx, tune, kind, bm, share):  # noqa: F811
         eye = torch.zeros(bm, IN_F, dtype=torch.bfloat16, device=DEV)
         eye[torch.arange(bm), start + torch.arange(bm)] = 1
         if kind == "dict":
-            y = bx.bf16x_gemm(eye, d["sign_packed"], d["mant_packed"], d["delta_packed"], d["emax"], OUT_F, IN_F,
-                              plan=plan, path="fused") if bm > 64 else few(bx, eye, d, plan)
+            y = product(bx, eye, d, OUT_F, IN_F, plan)
         else:
             y = bx.gguf.gguf_gemm_fused(eye, blocks, OUT_F, IN_F, ovf=t)
         assert np.array_equal(gpu_bits(y).T, bits[:, start:start + bm]), start
 
-
-def few(bx, x, d, plan):  # noqa: F811
-    """bf16x_gemm of the C ABI (up to 64 rows ops.bf16x_gemm takes the chunked kernel)."""
-    L, (ko, ke) = bx._lib.lib(), plan.kplan()
-    nb = L.bf16x_gemm_workspace(x.shape[0], OUT_F, IN_F)
-    ws = torch.empty(nb // 4 + 1, dtype=torch.int32, device=DEV)
-    y = torch.empty(x.shape[0], OUT_F, dtype=torch.bfloat16, device=DEV)
-    w = [v for k in ("sign_packed", "mant_packed", "delta_packed", "emax") for v in (d[k].data_ptr(), d[k].numel())]
-    assert L.bf16x_gemm(x.data_ptr(), bx._lib.BF16, x.shape[0], *w, ko.data_ptr(), ke.data_ptr(), OUT_F, IN_F, 16,
-                        bx._lib.EXACT, y.data_ptr(), bx._lib.BF16, ws.data_ptr(), nb,
-                        bx._lib.stream_of(x.device)) == 0
-    return y
