@@ -629,7 +629,6 @@ int bf16x_gemm_skinny_launch(const uint16_t* x, int64_t M, const uint32_t* s, co
                              int64_t in_f, bool exact, bool yf32, void* y, hipStream_t st);
 
 // streaming few-row kernel (gemm_stream.hip): M <= 16, no workspace
-bool bf16x_gemm_stream_fits(int64_t M, int64_t out_f, int64_t in_f, bool gg);
 int bf16x_gemm_stream_launch(const uint16_t* x, int64_t M, const uint32_t* s, const uint32_t* m, const uint32_t* d,
                              const uint16_t* e, const uint8_t* blocks, const uint32_t* kp_off, const uint32_t* kp_ent,
                              int64_t out_f, int64_t in_f, bool exact, bool yf32, void* y, hipStream_t st);

@@ -2,8 +2,9 @@
 // workgroups.
 //
 // Replaces _bf16x_gemm_fused_kernel / bf16x_fused_gemm (bf16x_gemm_fused.py:31-114)
-// for M of a few hundred rows and more: y[M, N] = x[M, K] . W[N, K]^T with W
-// decoded on the fly, fp32 accumulation.  SATURATED reproduces the reference
+// from tens of rows on: y[M, N] = x[M, K] . W[N, K]^T with W decoded on the
+// fly, fp32 accumulation (in four-step groups, K % 256 == 0, from 65 rows, or 33
+// of a weight of 2^25 elements; one step at a time from 192).  SATURATED reproduces the reference
 // kernel's numerics (code 7 -> exponent emax-7, bf16x_gemm_fused.py:84-87);
 // EXACT writes the overflow plan's entries over the decoded tile and
 // multiplies by the lossless weight.
@@ -17,9 +18,9 @@
 //    130-220 B/clk for 16-byte reads.  Register budget (two waves per SIMD,
 //    256 registers each) limits an MFMA wave to 128 accumulators.
 //
-// A workgroup is 8 waves (12 for the smaller tiles of the grouped kernel) and
-// owns an output tile of 256 x rows (tokens) by 128
-// W rows over a range of 64-column K steps (all of K, or one split of it when
+// A workgroup is 8 waves and owns an output tile of 256 x rows (tokens) by 128
+// W rows (the grouped kernel below also 128 or 64 by 128, with 12 waves) over a
+// range of 64-column K steps (all of K, or one split of it when
 // the tile count alone leaves CUs idle; split partials are fp32 and summed in
 // split order by a second kernel).
 //  * Waves 4-7 decode.  Wave 4+p decodes rows 32p .. 32p+31 of the W tile at
@@ -110,7 +111,7 @@ struct RawG {
 // share a W tile run on one XCD at the same time and share its L2.
 struct WsGrid {
   int mtiles, full, ltiles, lunits;
-  int bm;         // tokens per tile (kBM)
+  int bm;         // tokens per tile
 };
 struct WsWork {
   int64_t m0, n0;
@@ -483,8 +484,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // per atom, two decode waves), and launch, first loads and the partial tiles
 // are 9 us.  Two 64-row blocks per CU (16 waves) were no faster (M = 101: 49.8
 // against 49.8 us).  Calls against the tiled kernel these tiles replace:
-// 14336x4096 M = 101 66.7 -> 44 us, 4096x14336 66 -> 43.5, 6144x4096 40.5 ->
-// 28.5, 4096x4096 30.6 -> 23.3.
+// 14336x4096 M = 101 66.7 -> 44 us, 6144x4096 40.5 -> 28.5, 4096x4096 30.6 ->
+// 23.3; 4096x14336 59.6 -> 38.4 (on one weight, partly cached).
 // ---------------------------------------------------------------------------
 constexpr int kGroup = 4;                    // 64-column steps per group
 constexpr int kRowB4 = kGroup * kRowB;       // 512 bytes per tile row
@@ -750,7 +751,9 @@ void gemm_ws4_kernel(
     // XD steps (x) ahead, so an LDS read has at least eight MFMAs to arrive.
     // The group's last WQ quarters request the next group's operands: the
     // barrier comes before them, when all of this group's are in registers,
-    // which also frees the slot for the decode waves early.
+    // which also frees the slot for the decode waves early.  The ring fills
+    // the 168 registers: the 128-token kernel spills 1-2 of them and the
+    // two-term 64-token kernel 2-3 (8-16 bytes of scratch per lane).
     // NX = 2: x is two terms (hi, lo), both multiplied into the accumulator
     // (4096x4096 fp16 M = 64: 21.5 us for the call, 30.1 with the terms split
     // into 2 M rows and their results added by launches of their own).
@@ -807,7 +810,6 @@ void gemm_ws4_kernel(
     const int i = t / NJ, jj = t % NJ;
     acc[i][jj] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(X[i][q], wb[jj], acc[i][jj], 0, 0, 0);
   };
-#define BF16X_SG(mask, cnt) __builtin_amdgcn_sched_group_barrier(mask, cnt, 0)
 #define BF16X_SG(mask, cnt) __builtin_amdgcn_sched_group_barrier(mask, cnt, 0)
   bf16x8_t X0[NT][4], X1[NT][4], W0[NJ], W1[NJ];
   // step u of the group in `slot` (block step jx) with x in X; x of step
@@ -937,13 +939,13 @@ __global__ __launch_bounds__(256) void x_op_kernel(const void* __restrict__ x, i
 }
 
 // y over the split tiles: the sum of each element's fp32 partials in K-range
-// order (partial tile layout as ws_store writes it).  One thread per element
-// of the split tiles' 256 x 128 partials, in order.
+// order (partial tile layout as ws_store writes it), one thread per four
+// consecutive elements of the split tiles.
 template <int YT>
 __global__ __launch_bounds__(256) void ws_tile_reduce_kernel(const float* __restrict__ part, WsGrid g, int nsplit,
                                                              int64_t M, int64_t out_f, void* __restrict__ y,
                                                              bool yal) {
-  // four consecutive columns of one tile row per thread (kBN % 4 == 0): 16-byte
+  // four columns of one tile row (kBN % 4 == 0): 16-byte
   // partial loads, an 8-byte (bf16) or 16-byte (fp32) store when the row's
   // four outputs are in range and aligned (yal: y is 16-byte aligned)
   // (at most resident blocks x 256 x 128 elements: 32-bit indexes)
@@ -988,8 +990,8 @@ bool ws_grouped(int64_t in_f) {
   return (in_f / kStep) % kGroup == 0 && tuning(BF16X_TUNE_GEMM_WS_GROUPED) != 0;
 }
 
-// Resident blocks of the wave-specialised kernels: one per CU (128 KB of LDS
-// and 8 waves of 256 registers each); 256 CUs when there is no device to ask.
+// Resident blocks of the wave-specialised kernels: one per CU (128 KB of LDS,
+// and 8 waves of 256 registers or 12 of 168); 256 CUs when there is no device to ask.
 int64_t ws_resident() {
   static int64_t cache[64];
   int dev = 0, cus = 0;

@@ -10,10 +10,9 @@
 // Bound: the gathers.  An entry reads its code, sign, mantissa and emax from
 // four streams, and at one entry per ~38 elements nearly every cache line of
 // them is touched (84 MB at 14336x4096).  Measured there (1.55 M entries):
-// 13 + 4 + 16 us (15
-// + 4 + 18.5 with one entry of a thread in flight at a time), 48 us for the call
-// with its one wait for the count; the host builder, which
-// copies the streams back first, takes 30-40 ms.
+// 13 + 4 + 16 us (15 + 4 + 18.5 with one entry of a thread in flight at a
+// time), 48 us for the call with its one wait for the count; the host builder,
+// which copies the streams back first, takes 30-40 ms.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 

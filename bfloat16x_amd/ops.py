@@ -461,7 +461,7 @@ def bf16x_gemm(x, sign, mant, delta, emax, out_f, in_f, plan: Bf16xPlan | None =
     bf16x_gemm in the C ABI; one bf16 row the fused GEMV, bf16x_gemv);
     bf16 activations run one bf16 MFMA pass, fp16/fp32 activations are split
     as x = hi + lo (two bf16 terms, exact for fp16, 16 mantissa bits for
-    fp32), the rows of both in one launch, and added in fp32.
+    fp32) and summed in fp32 (see _gemm_terms).
     path "decode": W decoded into a temporary by the HIP decoder, then
     F.linear on the same device (fp32 for fp16/fp32 activations).
     path "auto": "decode" from GEMM_DECODE_MIN_ROWS rows on (_TALL / _WIDE for

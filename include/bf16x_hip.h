@@ -26,9 +26,11 @@
  *      tile_ent uint32 [n_fix]        (column within tile << 16) | exact bf16 bits
  *      tile_sat uint8  [n_fix]        saturated exponent max(emax - 7, 0) of the
  *                                     entry's element (used by the GEMV overlay)
- *    Built by bf16x_plan_host() or bf16x_plan_from_csr().
+ *    Built by bf16x_plan_host(), bf16x_plan_device_count() / _write() or
+ *    bf16x_plan_from_csr().
  *  - All device work is enqueued on `stream` (a hipStream_t; NULL = the
- *    default stream) and is asynchronous.
+ *    default stream) and is asynchronous.  The current device must be the one
+ *    that the pointers and the stream belong to.
  *  - Return value: 0 = success, < 0 = invalid argument (see BF16X_E*),
  *    > 0 = a hipError_t reported by the runtime.
  *  - Entry points keep no state between calls, and concurrent calls on
