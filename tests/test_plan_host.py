@@ -39,6 +39,7 @@ def test_device_builder_runs_on_the_dicts_gpu(monkeypatch):
     _lib.lib()
     monkeypatch.setattr(codec, "_on_device", lambda packed, device: True)
     monkeypatch.setattr(torch.cuda, "device", guard)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
     monkeypatch.setattr(_lib, "lib", lambda stub=Lib(): stub)
     monkeypatch.setattr(_lib, "stream_of", lambda dev: seen.append(("stream", current[0])) or 0)
     plan = bx.build_plan_host(d, device="cuda:1")
