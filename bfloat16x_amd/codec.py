@@ -274,6 +274,14 @@ def build_plan_host(packed: dict, check: int = 1, device=None) -> Bf16xPlan:
     return plan.to(device) if device is not None else plan
 
 
+def _csr_offsets(oloff: torch.Tensor, n: int) -> torch.Tensor:
+    """Row offsets held in [0, n] and ascending, whatever the caller's CSR: the
+    kernels read entries [off[r], off[r + 1]) of a row, and the regrouped plans
+    (kplan, cplan) have room for n entries, which offsets that fall back would
+    count twice."""
+    return torch.cummax(oloff.reshape(-1).clamp(0, n), 0).values.contiguous()
+
+
 def build_plan_from_csr(olk, old, oloff, sign, mant, emax, out_f: int, in_f: int) -> Bf16xPlan:
     """Plan from the reference's device CSR (bf16x_fused.py:165-179): the
     offsets are reused as tile offsets, entries are re-encoded on the GPU."""
@@ -283,8 +291,9 @@ def build_plan_from_csr(olk, old, oloff, sign, mant, emax, out_f: int, in_f: int
             raise ValueError(f"{nm} must be an int32 tensor on the streams' GPU ({dev})")
     if oloff.numel() != int(out_f) + 1 or old.numel() != olk.numel():
         raise ValueError("CSR shape: oloff needs out_f + 1 offsets and old one value per olk column")
-    olk, old, oloff = olk.contiguous(), old.contiguous(), oloff.contiguous()
+    olk, old = olk.contiguous(), old.contiguous()
     n = int(olk.numel())
+    oloff = _csr_offsets(oloff, n)
     ent = torch.zeros(max(n, 1), dtype=torch.int32, device=dev)
     sat = torch.zeros(max(n, 1), dtype=torch.uint8, device=dev)
     st = _lib.lib().bf16x_plan_from_csr(_lib.ptr(olk), _lib.ptr(old),
@@ -292,9 +301,7 @@ def build_plan_from_csr(olk, old, oloff, sign, mant, emax, out_f: int, in_f: int
                                         int(out_f), int(in_f), n, ent.data_ptr(), sat.data_ptr(),
                                         _lib.stream_of(dev))
     _lib.check(st, "bf16x_plan_from_csr")
-    # the kernels read entries [off[r], off[r + 1]) of a row: offsets held in
-    # [0, n] keep every read inside the entry arrays whatever the caller's CSR
-    return Bf16xPlan(oloff.clamp(0, n), ent, sat, n, int(out_f), int(in_f))
+    return Bf16xPlan(oloff, ent, sat, n, int(out_f), int(in_f))
 
 
 def build_plan_device(ovf_idx, ovf_val, sign, mant, emax, out_f: int, in_f: int) -> Bf16xPlan:

@@ -91,6 +91,31 @@ def test_kplan_out_of_order(bx, kind):  # noqa: F811
     assert np.array_equal(kp_ent[:ref_ent.size], ref_ent)
 
 
+# a CSR whose offsets fall back: its plan's rows share no entry, so the
+# regrouped plans stay inside their n entries; a well-formed one is unchanged
+@pytest.mark.parametrize("kind", ["ascending", "falling", "out of range"])
+def test_csr_offsets(bx, kind):  # noqa: F811
+    out_f, in_f = 64, 512
+    d = bx.bf16x_quantize(torch.randn(out_f, in_f, generator=torch.Generator().manual_seed(1)).to(DEV))
+    off, cols, _ = make_plan(out_f, in_f, 9, 4)
+    n, good = cols.size, off.astype(np.int32)
+    bad = good.copy()
+    if kind == "falling":
+        bad[1::2] = n
+        bad[2::2] = 0
+    elif kind == "out of range":
+        bad[10], bad[20], bad[30] = -7, 2 ** 30, 3
+    to = lambda a: torch.from_numpy(a.astype(np.int32)).to(DEV)
+    plan = bx.codec.build_plan_from_csr(to(cols), torch.full((n,), 9, dtype=torch.int32, device=DEV), to(bad),
+                                        d["sign_packed"], d["mant_packed"], d["emax"], out_f, in_f)
+    t = plan.tile_off.cpu().numpy()
+    assert t.min() >= 0 and t.max() <= n and np.all(np.diff(t) >= 0)
+    assert kind != "ascending" or np.array_equal(t, good)
+    for o, e in (plan.kplan(), plan.cplan()):
+        assert 0 <= int(o[-1]) <= n <= e.numel()
+    torch.cuda.synchronize()
+
+
 # the scan at its tile's edges and with more tiles than one pass over their
 # first elements takes (1024), through the chunk plan's offsets
 @pytest.mark.parametrize("out_f,in_f", [(1, 256), (4095, 256), (4096, 256), (4097, 256), (8192, 256), (140000, 8192)])

@@ -1,8 +1,9 @@
-"""CPU test of how the device plan builder is reached: with the dict's GPU as
-the current device, whatever was current before."""
+"""CPU tests around the device plan builders: the dict's GPU is the current
+device while one runs, and a CSR's offsets cover no entry twice."""
 import contextlib
 import ctypes
 
+import pytest
 import torch
 
 import bfloat16x_amd as bx
@@ -46,3 +47,16 @@ def test_device_builder_runs_on_the_dicts_gpu(monkeypatch):
     where = d["delta_ovf_idx"].device
     assert seen == [("stream", where), ("count", where), ("write", where)]
     assert plan.n_fix == 0 and current == ["another"]
+
+
+@pytest.mark.parametrize("off", [[0, 3, 3, 7, 9], [0, 9, 0, 9, 9], [-5, 4, 2, 100, 1], [9, 0, 0, 0, 0], [0, 0, 0, 0, 0]])
+def test_csr_offsets_cover_no_entry_twice(off):
+    """Well-formed offsets stay; others become ascending inside [0, n], so the
+    rows' entries together are at most n."""
+    n = 9
+    got = codec._csr_offsets(torch.tensor(off, dtype=torch.int32), n)
+    assert got.dtype == torch.int32 and got.is_contiguous() and got.numel() == len(off)
+    d = got.diff()
+    assert int(got.min()) >= 0 and int(got.max()) <= n and bool((d >= 0).all()) and int(d.sum()) <= n
+    if sorted(off) == off:
+        assert got.tolist() == off
